@@ -102,6 +102,7 @@ __device__ __forceinline__ void q4k_stage_tile(const float *__restrict__ x, floa
 }
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t axh_u32u __attribute__((aligned(2))); // a dword at a 2-byte aligned address
 
 // 16-byte weight load; kNT marks it non-temporal (streamed once per call).
 template <bool kNT>
@@ -2420,112 +2421,157 @@ extern "C" __global__ void __launch_bounds__(64)
 }
 
 // ===========================================================================
-// Decode-only kernels (bit-exact checks of the dequantised weights)
+// Decode-only kernels (whole tensors to f32, bit-exact)
 // ===========================================================================
-// Q5_K: one thread per (superblock, 16-byte qs slice), as Q4_K plus the
-// fifth bit from qh: fma(d*sc, q, -(dmin*m)) with d*sc, dmin*m and (d*sc)*q
-// exact in f32 (q <= 31), so the one rounding is the subtraction's.
-extern "C" __global__ void __launch_bounds__(256)
-    axh_q5k_dequant(const uint8_t *__restrict__ q, float *__restrict__ w, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
-  const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
-  const uint32_t sb = gid >> 3, k = gid & 7u, c = k >> 1, h = k & 1u;
-  if (sb >= a.n_units) return;
-  const uint8_t *b = q + (size_t)sb * kQ5kSbBytes;
-  const uint4 hd = *reinterpret_cast<const uint4 *>(b);
-  const uint4 qv = *reinterpret_cast<const uint4 *>(b + 48u + 16u * k);
-  const uint4 hv = *reinterpret_cast<const uint4 *>(b + 16u + 16u * h);
-  uint32_t scp, mp;
-  q4k_scale_min_pair(hd.y, hd.z, hd.w, c, &scp, &mp);
-  const float d = f16_to_f32(hd.x & 0xFFFFu), dmin = f16_to_f32(hd.x >> 16);
-  const float d1 = d * (float)(scp & 0xFFu), m1f = dmin * (float)(mp & 0xFFu);
-  const float d2 = d * (float)(scp >> 8), m2f = dmin * (float)(mp >> 8);
-  float *wl = w + (size_t)sb * kQ4kSbElems + 64u * c + 16u * h;
-  float *wh = wl + 32;
-  const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
-  const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w};
+// Bound by the f32 store stream (4 B per weight against 0.56-0.82 B read), so
+// each thread decodes one dword of 4 low and 4 high nibbles (Q6_K: 4 values of
+// each of a half's four parts) and 8 neighbouring threads store 128
+// consecutive bytes per instruction.  4096 x 14336, us per call, against one
+// 64-byte run per thread (every lane of a store 64 bytes from the next): Q4_K
+// 38.3 vs 78.9 (7.0 TB/s), Q5_K 39.2 vs 84.7, Q6_K 40.8 vs 121.0, Q4_0 38.4 vs
+// 92.9.
+typedef float axh_f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// kDqUnits units per thread (a workgroup walks consecutive units), their loads
+// ahead of the first store; stores non-temporal, as nothing here reads w back.
+// Q4_K at 4096 x 14336: 38.3 us with 2 units, 44.2 with 1, 42.3 with 4; 50.0
+// with 2 units and cached stores.
+constexpr int kDqUnits = 2;
+
+// Four nibbles (bits kShift.. of each byte of w) as fma(d, nibble, -m).
+template <int kShift>
+__device__ __forceinline__ f32x4_t dq_nibbles(uint32_t w, float d, float m) {
+  f32x4_t v;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    float lo[4], hi[4];
+  for (int e = 0; e < 4; ++e)
+    v[e] = __builtin_fmaf(d, (float)((w >> (8 * e + kShift)) & 15u), -m);
+  return v;
+}
+
+// Q4_K and Q5_K: thread (superblock, qs dword t of chunk c).  Each value is
+// fma(d*sc, q, -(dmin*m)): d*sc, dmin*m and (d*sc)*q are exact in f32, so the
+// single rounding equals the reference's d1*lo - m1f.  Q5_K adds the fifth
+// bits: bit 2c of qh byte l for weight 64c + l, bit 2c + 1 for 64c + 32 + l.
+template <bool kQ5>
+__device__ __forceinline__ void q45k_dequant(const uint8_t *__restrict__ q, float *__restrict__ w,
+                                             uint32_t n_sb) {
+  constexpr uint32_t kBytes = kQ5 ? kQ5kSbBytes : kQ4kSbBytes;
+  const uint32_t k = threadIdx.x & 31u, c = k >> 3, t = k & 7u;
+  const uint32_t sb0 = blockIdx.x * (8u * kDqUnits) + (threadIdx.x >> 5);
+  uint4 hd[kDqUnits];
+  uint32_t qv[kDqUnits], hv[kDqUnits];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t byte = (qw[t] >> (8 * e)) & 0xFFu, bits = (hw[t] >> (8 * e + 2 * c)) & 3u;
-      lo[e] = __builtin_fmaf(d1, (float)((byte & 15u) + 16u * (bits & 1u)), -m1f);
-      hi[e] = __builtin_fmaf(d2, (float)((byte >> 4) + 16u * (bits >> 1)), -m2f);
+  for (int u = 0; u < kDqUnits; ++u) {
+    const uint32_t sb = min(sb0 + 8u * (uint32_t)u, n_sb - 1u);
+    const uint8_t *b = q + (size_t)sb * kBytes;
+    hd[u] = *reinterpret_cast<const uint4 *>(b);
+    qv[u] = *reinterpret_cast<const uint32_t *>(b + (kQ5 ? 48u : 16u) + 4u * k);
+    if constexpr (kQ5) hv[u] = *reinterpret_cast<const uint32_t *>(b + 16u + 4u * t) >> (2u * c);
+  }
+#pragma unroll
+  for (int u = 0; u < kDqUnits; ++u) {
+    const uint32_t sb = sb0 + 8u * (uint32_t)u;
+    if (sb >= n_sb) return;
+    uint32_t scp, mp;
+    q4k_scale_min_pair(hd[u].y, hd[u].z, hd[u].w, c, &scp, &mp);
+    const float d = f16_to_f32(hd[u].x & 0xFFFFu), dmin = f16_to_f32(hd[u].x >> 16);
+    const float d1 = d * (float)(scp & 0xFFu), m1 = dmin * (float)(mp & 0xFFu);
+    const float d2 = d * (float)(scp >> 8), m2 = dmin * (float)(mp >> 8);
+    f32x4_t lo, hi;
+    if constexpr (kQ5) {
+      const uint32_t l5 = (qv[u] & 0x0F0F0F0Fu) | ((hv[u] & 0x01010101u) << 4);
+      const uint32_t h5 = ((qv[u] >> 4) & 0x0F0F0F0Fu) | ((hv[u] & 0x02020202u) << 3);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = __builtin_fmaf(d1, (float)((l5 >> (8 * e)) & 0xFFu), -m1);
+        hi[e] = __builtin_fmaf(d2, (float)((h5 >> (8 * e)) & 0xFFu), -m2);
+      }
+    } else {
+      lo = dq_nibbles<0>(qv[u], d1, m1);
+      hi = dq_nibbles<4>(qv[u], d2, m2);
     }
-    *reinterpret_cast<float4 *>(wl + 4 * t) = make_float4(lo[0], lo[1], lo[2], lo[3]);
-    *reinterpret_cast<float4 *>(wh + 4 * t) = make_float4(hi[0], hi[1], hi[2], hi[3]);
+    f32x4_t *o = reinterpret_cast<f32x4_t *>(w + (size_t)sb * kQ4kSbElems + 64u * c + 4u * t);
+    __builtin_nontemporal_store(lo, o);
+    __builtin_nontemporal_store(hi, o + 8);
   }
 }
 
-// Q6_K: one thread per (superblock, half n, part p): 32 weights
-// d * sc * (q - 32), exact in f32.  Byte reads (superblocks are 2-byte aligned).
-extern "C" __global__ void __launch_bounds__(256)
-    axh_q6k_dequant(const uint8_t *__restrict__ q, float *__restrict__ w, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
-  const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
-  const uint32_t sb = gid >> 3, n = (gid >> 2) & 1u, p = gid & 3u;
-  if (sb >= a.n_units) return;
-  const uint8_t *b = q + (size_t)sb * kQ6kSbBytes;
-  const float d = f16_to_f32((uint32_t)b[208] | ((uint32_t)b[209] << 8));
-  const float s0 = d * (float)(int8_t)b[192u + 8u * n + 2u * p];
-  const float s1 = d * (float)(int8_t)b[192u + 8u * n + 2u * p + 1u];
-  const uint8_t *ql = b + 64u * n + 32u * (p & 1u), *qh = b + 128u + 32u * n;
-  float *o = w + (size_t)sb * kQ4kSbElems + 128u * n + 32u * p;
-  for (uint32_t l = 0; l < 32; ++l) {
-    const uint32_t v = ((ql[l] >> (4u * (p >> 1))) & 15u) | (((qh[l] >> (2u * p)) & 3u) << 4);
-    o[l] = (l < 16 ? s0 : s1) * (float)((int)v - 32);
-  }
-}
-
-// Q4_K: one thread per (superblock, 16-byte qs slice).  Each value is
-// fma(d*sc, nibble, -(dmin*m)): d*sc, dmin*m and (d*sc)*nibble are exact in
-// f32, so the single rounding equals the reference's d1*lo - m1f.
 extern "C" __global__ void __launch_bounds__(256)
     axh_q4k_dequant(const uint8_t *__restrict__ q, float *__restrict__ w, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
-  const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
-  const uint32_t sb = gid >> 3, k = gid & 7u, c = k >> 1, h = k & 1u;
-  if (sb >= a.n_units) return;
-  const uint8_t *b = q + (size_t)sb * kQ4kSbBytes;
-  const uint4 hd = *reinterpret_cast<const uint4 *>(b);
-  const uint4 qv = *reinterpret_cast<const uint4 *>(b + 16u + 16u * k);
-  uint32_t scp, mp;
-  q4k_scale_min_pair(hd.y, hd.z, hd.w, c, &scp, &mp);
-  const float d = f16_to_f32(hd.x & 0xFFFFu), dmin = f16_to_f32(hd.x >> 16);
-  const float d1 = d * (float)(scp & 0xFFu), m1f = dmin * (float)(mp & 0xFFu);
-  const float d2 = d * (float)(scp >> 8), m2f = dmin * (float)(mp >> 8);
-  float *wl = w + (size_t)sb * kQ4kSbElems + 64u * c + 16u * h;
-  float *wh = wl + 32;
-  const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
+  q45k_dequant<false>(q, w, a.n_units);
+}
+
+extern "C" __global__ void __launch_bounds__(256)
+    axh_q5k_dequant(const uint8_t *__restrict__ q, float *__restrict__ w, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
+  q45k_dequant<true>(q, w, a.n_units);
+}
+
+// Q6_K: thread (superblock, half n, l = 4t ..), d * sc * (q - 32), exact in
+// f32: 4 weights of each of the half's four 32-weight parts.  Superblocks are
+// 2-byte and w 4-byte aligned.
+extern "C" __global__ void __launch_bounds__(256)
+    axh_q6k_dequant(const uint8_t *__restrict__ q, float *__restrict__ w, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
+  const uint32_t k = threadIdx.x & 15u, n = k >> 3, t = k & 7u;
+  const uint32_t sb0 = blockIdx.x * (16u * kDqUnits) + (threadIdx.x >> 4);
+  uint32_t q0[kDqUnits], q1[kDqUnits], qh[kDqUnits], sc[kDqUnits][2], d16[kDqUnits];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    float4 lo, hi;
-    lo.x = __builtin_fmaf(d1, (float)((qw[t] >> 0) & 15u), -m1f);
-    lo.y = __builtin_fmaf(d1, (float)((qw[t] >> 8) & 15u), -m1f);
-    lo.z = __builtin_fmaf(d1, (float)((qw[t] >> 16) & 15u), -m1f);
-    lo.w = __builtin_fmaf(d1, (float)((qw[t] >> 24) & 15u), -m1f);
-    hi.x = __builtin_fmaf(d2, (float)((qw[t] >> 4) & 15u), -m2f);
-    hi.y = __builtin_fmaf(d2, (float)((qw[t] >> 12) & 15u), -m2f);
-    hi.z = __builtin_fmaf(d2, (float)((qw[t] >> 20) & 15u), -m2f);
-    hi.w = __builtin_fmaf(d2, (float)((qw[t] >> 28) & 15u), -m2f);
-    *reinterpret_cast<float4 *>(wl + 4 * t) = lo;
-    *reinterpret_cast<float4 *>(wh + 4 * t) = hi;
+  for (int u = 0; u < kDqUnits; ++u) {
+    const uint32_t sb = min(sb0 + 16u * (uint32_t)u, a.n_units - 1u);
+    const uint8_t *b = q + (size_t)sb * kQ6kSbBytes;
+    q0[u] = *reinterpret_cast<const axh_u32u *>(b + 64u * n + 4u * t);
+    q1[u] = *reinterpret_cast<const axh_u32u *>(b + 64u * n + 32u + 4u * t);
+    qh[u] = *reinterpret_cast<const axh_u32u *>(b + 128u + 32u * n + 4u * t);
+    sc[u][0] = *reinterpret_cast<const axh_u32u *>(b + 192u + 8u * n);
+    sc[u][1] = *reinterpret_cast<const axh_u32u *>(b + 196u + 8u * n);
+    d16[u] = *reinterpret_cast<const uint16_t *>(b + 208u);
+  }
+#pragma unroll
+  for (int u = 0; u < kDqUnits; ++u) {
+    const uint32_t sb = sb0 + 16u * (uint32_t)u;
+    if (sb >= a.n_units) return;
+    const float d = f16_to_f32(d16[u]);
+    float *o = w + (size_t)sb * kQ4kSbElems + 128u * n + 4u * t;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t v = (((p & 1 ? q1[u] : q0[u]) >> (p & 2 ? 4 : 0)) & 0x0F0F0F0Fu) |
+                         (((qh[u] >> (2 * p)) & 0x03030303u) << 4);
+      // scale of weights 32p + 16 (t / 4) ..: byte 2p + t / 4 of the half's eight
+      const uint32_t by = (sc[u][p >> 1] >> (16 * (p & 1) + 8u * (t >> 2))) & 0xFFu;
+      const float s = d * (float)(int8_t)by;
+      axh_f4u r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = s * ((float)((v >> (8 * e)) & 0xFFu) - 32.0f);
+      __builtin_nontemporal_store(r, reinterpret_cast<axh_f4u *>(o + 32 * p));
+    }
   }
 }
 
-// Q4_0: one thread per block; (nibble - 8) * d is exact in f32.
+// Q4_0: thread (block, output float4 t): the low nibbles of qs dword t, or the
+// high nibbles of dword t - 4; (nibble - 8) * d is exact in f32.  A wave's
+// store covers 1 KiB.  Blocks are 2-byte and w 4-byte aligned.
+constexpr int kDq0Units = 4;
 extern "C" __global__ void __launch_bounds__(256)
     axh_q4_0_dequant(const uint8_t *__restrict__ q, float *__restrict__ w, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
-  const uint32_t blk = blockIdx.x * 256u + threadIdx.x;
-  if (blk >= a.n_units) return;
-  const uint16_t *p16 = reinterpret_cast<const uint16_t *>(q + (size_t)blk * kQ4_0BlockBytes);
-  const float d = f16_to_f32(p16[0]);
-  float *wb = w + (size_t)blk * kQ4_0BlockElems;
+  const uint32_t t = threadIdx.x & 7u;
+  const uint32_t b0 = blockIdx.x * (32u * kDq0Units) + (threadIdx.x >> 3);
+  uint32_t qv[kDq0Units], d16[kDq0Units];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t two = p16[1 + i]; // qs bytes 2i, 2i+1
-    wb[2 * i] = ((float)(two & 15u) - 8.0f) * d;
-    wb[2 * i + 1] = ((float)((two >> 8) & 15u) - 8.0f) * d;
-    wb[16 + 2 * i] = ((float)((two >> 4) & 15u) - 8.0f) * d;
-    wb[16 + 2 * i + 1] = ((float)((two >> 12) & 15u) - 8.0f) * d;
+  for (int u = 0; u < kDq0Units; ++u) {
+    const uint32_t blk = min(b0 + 32u * (uint32_t)u, a.n_units - 1u);
+    const uint8_t *b = q + (size_t)blk * kQ4_0BlockBytes;
+    d16[u] = *reinterpret_cast<const uint16_t *>(b);
+    qv[u] = *reinterpret_cast<const axh_u32u *>(b + 2u + 4u * (t & 3u)) >> (t & 4u);
+  }
+#pragma unroll
+  for (int u = 0; u < kDq0Units; ++u) {
+    const uint32_t blk = b0 + 32u * (uint32_t)u;
+    if (blk >= a.n_units) return;
+    const float d = f16_to_f32(d16[u]);
+    axh_f4u v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = ((float)((qv[u] >> (8 * e)) & 15u) - 8.0f) * d;
+    __builtin_nontemporal_store(
+        v, reinterpret_cast<axh_f4u *>(w + (size_t)blk * kQ4_0BlockElems + 4u * t));
   }
 }
 

@@ -1891,50 +1891,56 @@ axh_status axh_q4k_matmul_f32(axh_context *ctx, const void *q, const float *x, u
   return axh_q4k_matmul_f16(ctx, q, x16, y, n_rows, sb_per_row, batch, variant, stream);
 }
 
+// One launch of 256-thread workgroups over n_units units, units_per_wg each.
 static axh_status count_launch(axh_context *ctx, const char *name, const void *in, void *out,
-                               uint64_t n_threads, uint64_t n_units, void *stream) {
+                               uint32_t units_per_wg, uint64_t n_units, void *stream) {
   if (!ctx) return fail(AXH_ERR_INVALID_ARGUMENT, "ctx is NULL");
   if (n_units == 0) return ok();
   if (!in || !out) return fail(AXH_ERR_INVALID_ARGUMENT, "NULL device pointer");
-  if (n_units > 0xFFFFFFFFull || n_threads > (uint64_t)0xFFFFFFFFull * 256ull)
+  if (n_units > 0xFFFFFFFFull)
     return fail(AXH_ERR_INVALID_ARGUMENT, "too many units for one launch");
   axh_kernel *k = nullptr;
   axh_status s = builtin_kernel(ctx, name, 2, sizeof(CountArgs), 256, &k);
   if (s != AXH_OK) return s;
   CountArgs a{(uint32_t)n_units};
-  const uint32_t grid[3] = {(uint32_t)((n_threads + 255u) / 256u), 1, 1};
+  const uint32_t grid[3] = {(uint32_t)((n_units + units_per_wg - 1u) / units_per_wg), 1, 1};
   void *bufs[2] = {const_cast<void *>(in), out};
   hipSetDevice(ctx->core->device);
   s = launch_raw(k, grid, bufs, 2, &a, sizeof(a), 0, pick_stream(ctx, stream));
   return s == AXH_OK ? ok() : s;
 }
 
+// Units a thread of the decode kernels takes (kDqUnits and kDq0Units in
+// q4_matvec.hip); 32 threads per Q4_K / Q5_K superblock, 16 per Q6_K
+// superblock, 8 per Q4_0 block.
+static constexpr uint32_t kDqUnits = 2, kDq0Units = 4;
+
 axh_status axh_q5k_dequant(axh_context *ctx, const void *q, float *w, uint64_t n_sb, void *stream) {
   if (n_sb > (1ull << 28)) return fail(AXH_ERR_INVALID_ARGUMENT, "too many superblocks");
   if (((uintptr_t)q & 15u) || ((uintptr_t)w & 15u))
     return fail(AXH_ERR_INVALID_ARGUMENT, "q and w must be 16-byte aligned");
-  return count_launch(ctx, "axh_q5k_dequant", q, w, n_sb * 8u, n_sb, stream);
+  return count_launch(ctx, "axh_q5k_dequant", q, w, 8u * kDqUnits, n_sb, stream);
 }
 
 axh_status axh_q6k_dequant(axh_context *ctx, const void *q, float *w, uint64_t n_sb, void *stream) {
   if (n_sb > (1ull << 28)) return fail(AXH_ERR_INVALID_ARGUMENT, "too many superblocks");
   if ((uintptr_t)q & 1u) return fail(AXH_ERR_INVALID_ARGUMENT, "q must be 2-byte aligned");
   if ((uintptr_t)w & 3u) return fail(AXH_ERR_INVALID_ARGUMENT, "w must be 4-byte aligned");
-  return count_launch(ctx, "axh_q6k_dequant", q, w, n_sb * 8u, n_sb, stream);
+  return count_launch(ctx, "axh_q6k_dequant", q, w, 16u * kDqUnits, n_sb, stream);
 }
 
 axh_status axh_q4k_dequant(axh_context *ctx, const void *q, float *w, uint64_t n_sb, void *stream) {
   if (n_sb > (1ull << 28)) return fail(AXH_ERR_INVALID_ARGUMENT, "too many superblocks");
   if (((uintptr_t)q & 15u) || ((uintptr_t)w & 15u))
     return fail(AXH_ERR_INVALID_ARGUMENT, "q and w must be 16-byte aligned");
-  return count_launch(ctx, "axh_q4k_dequant", q, w, n_sb * 8u, n_sb, stream);
+  return count_launch(ctx, "axh_q4k_dequant", q, w, 8u * kDqUnits, n_sb, stream);
 }
 
 axh_status axh_q4_0_dequant(axh_context *ctx, const void *q, float *w, uint64_t n_blocks,
                             void *stream) {
   if (((uintptr_t)q & 1u) || ((uintptr_t)w & 3u))
     return fail(AXH_ERR_INVALID_ARGUMENT, "q must be 2-byte and w 4-byte aligned");
-  return count_launch(ctx, "axh_q4_0_dequant", q, w, n_blocks, n_blocks, stream);
+  return count_launch(ctx, "axh_q4_0_dequant", q, w, 32u * kDq0Units, n_blocks, stream);
 }
 
 // Measurement helpers: the matvec's launch shape (one 512-thread workgroup
@@ -2001,14 +2007,14 @@ axh_status axh_launch_empty(axh_context *ctx, uint32_t *out, uint32_t out_words,
 uint32_t axh_cu_count(axh_context *ctx) { return ctx ? ctx->core->cu_count : 0u; }
 
 axh_status axh_f16_widen(axh_context *ctx, const uint16_t *h, float *f, uint64_t n, void *stream) {
-  return count_launch(ctx, "axh_f16_widen", h, f, n, n, stream);
+  return count_launch(ctx, "axh_f16_widen", h, f, 256u, n, stream);
 }
 
 axh_status axh_f32_to_f16(axh_context *ctx, const float *x, uint16_t *h, uint64_t n, void *stream) {
   if (n > 0xFFFFFFF0ull) return fail(AXH_ERR_INVALID_ARGUMENT, "n too large for one launch");
   if (((uintptr_t)x & 15u) || ((uintptr_t)h & 15u))
     return fail(AXH_ERR_INVALID_ARGUMENT, "x and h must be 16-byte aligned");
-  return count_launch(ctx, "axh_f32_to_f16", x, h, (n + 7u) / 8u, n, stream);
+  return count_launch(ctx, "axh_f32_to_f16", x, h, 2048u, n, stream);
 }
 
 } // extern "C"
