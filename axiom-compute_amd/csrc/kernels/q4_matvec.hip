@@ -2048,16 +2048,73 @@ AXH_Q4K_MATVEC_COLS(4, 8, 0, 1)
 // n_superblocks: u32 @0; @workgroup(64,1,1); dispatched as 1x1x1).  One wave
 // computes y[0]; workgroups other than 0 return, like the reference's
 // `if gid(0) >= 1 { return; }`.
-constexpr uint32_t kRefTileSb = 16; // 17 KiB static LDS tile
-extern "C" __global__ void __launch_bounds__(64)
+// The one wave meets no x value twice, so x goes straight to registers: lane
+// 8g + k takes superblock 8 it + g and its qs bytes [16k, 16k + 16) with the
+// 32 x values they meet, kRefAhead iterations of ten 16-byte loads in flight
+// (60 of the load counter's 63): the kernel is bound by the latency of one
+// wave's loads, and by its VALU work once those are covered.  512 superblocks
+// took 94 us with x staged through a 16-superblock LDS tile.
+constexpr int kRefAhead = 6;
+__device__ __forceinline__ float sum16(const float4 (&v)[4]) {
+  return (((v[0].x + v[0].y) + (v[0].z + v[0].w)) + ((v[1].x + v[1].y) + (v[1].z + v[1].w))) +
+         (((v[2].x + v[2].y) + (v[2].z + v[2].w)) + ((v[3].x + v[3].y) + (v[3].z + v[3].w)));
+}
+extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
     q4km_dequant_matvec(const uint8_t *__restrict__ q, const float *__restrict__ x,
                         float *__restrict__ y, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
-  __shared__ float lds[kRefTileSb * 256 + kRefTileSb * 16];
   if (blockIdx.x != 0 || blockIdx.y != 0 || blockIdx.z != 0) return;
-  if (a.n_units <= kRefTileSb)
-    q4k_matvec_body<1, 1, 2, false, false>(q, x, y, 1u, a.n_units, kRefTileSb, 0u, lds);
-  else
-    q4k_matvec_body<1, 1, 2, false, true>(q, x, y, 1u, a.n_units, kRefTileSb, 0u, lds);
+  const uint32_t lane = threadIdx.x, nsb = a.n_units;
+  if (nsb == 0) { // the reference returns +0.0 (AT-1323)
+    if (lane == 0) y[0] = 0.0f;
+    return;
+  }
+  const uint32_t g = lane >> 3, k = lane & 7u, c = k >> 1;
+  uint4 hd[kRefAhead], qv[kRefAhead];
+  float4 xl[kRefAhead][4], xh[kRefAhead][4];
+  auto load = [&](int p, uint32_t it) { // past the last superblock: the last one again
+    const uint32_t sb = min(it * 8u + g, nsb - 1u);
+    const uint8_t *b = q + (size_t)sb * kQ4kSbBytes;
+    hd[p] = load16<false>(b);
+    qv[p] = load16<false>(b + 16u + 16u * k);
+    const float4 *xp =
+        reinterpret_cast<const float4 *>(x + (size_t)sb * 256u + 64u * c + 16u * (k & 1u));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      xl[p][t] = xp[t];
+      xh[p][t] = xp[8 + t];
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < kRefAhead; ++p) load(p, (uint32_t)p);
+  __builtin_amdgcn_sched_barrier(0);
+  const uint32_t n_it = (nsb + 7u) >> 3;
+  float acc = 0.0f;
+  for (uint32_t it0 = 0; it0 < n_it; it0 += kRefAhead) {
+#pragma unroll
+    for (int p = 0; p < kRefAhead; ++p) {
+      const uint32_t it = it0 + (uint32_t)p;
+      uint32_t scp, mp;
+      q4k_scale_min_pair(hd[p].y, hd[p].z, hd[p].w, c, &scp, &mp);
+      const float d = f16_to_f32(hd[p].x & 0xFFFFu), dmin = f16_to_f32(hd[p].x >> 16);
+      float alo = 0.0f, ahi = 0.0f;
+      q4k_dword(qv[p].x, xl[p][0], xh[p][0], alo, ahi);
+      q4k_dword(qv[p].y, xl[p][1], xh[p][1], alo, ahi);
+      q4k_dword(qv[p].z, xl[p][2], xh[p][2], alo, ahi);
+      q4k_dword(qv[p].w, xl[p][3], xh[p][3], alo, ahi);
+      const float sc0 = (float)(scp & 0xFFu) * 16777216.0f; // 2^24
+      const float sc1 = (float)(scp >> 8) * 1048576.0f;     // 2^20
+      const float m0 = (float)(mp & 0xFFu), m1 = (float)(mp >> 8);
+      const float dot = __builtin_fmaf(sc0, alo, sc1 * ahi);
+      const float mins = __builtin_fmaf(m0, sum16(xl[p]), m1 * sum16(xh[p]));
+      const float v = __builtin_fmaf(d, dot, __builtin_fmaf(-dmin, mins, acc));
+      acc = it * 8u + g < nsb ? v : acc;
+      __builtin_amdgcn_sched_barrier(0); // the loads stay ahead of the next compute
+      load(p, it + kRefAhead);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  const float r = wave_sum(acc);
+  if (lane == 0) y[0] = r;
 }
 
 // ===========================================================================
@@ -2407,17 +2464,66 @@ AXH_Q4_0_MATVEC_ONEP(16)
 
 // Reference-compatible entry point for examples/q4_0_dequant_matvec.axc
 // (bindings q=0, x=1, y=2; push constant n_blocks: u32 @0; 1x1x1 of 64).
-constexpr uint32_t kRefTileB = 128; // 17 KiB static LDS tile
-extern "C" __global__ void __launch_bounds__(64)
+// As q4km_dequant_matvec: x straight to registers.  Lane 4i + t takes dword t
+// of the qs of block 16u + i and its two float4 of x, so that every load of
+// the wave covers whole blocks; 64 blocks per iteration, kRef0Ahead
+// iterations in flight.
+constexpr int kRef0Ahead = 4;
+struct Ref0Iter {
+  uint32_t d[4], qv[4];
+  float4 xl[4], xh[4];
+};
+extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
     q4_0_dequant_matvec(const uint8_t *__restrict__ q, const float *__restrict__ x,
                         float *__restrict__ y, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
-  __shared__ float lds[(kRefTileB / 2) * 64 + kRefTileB];
   if (blockIdx.x != 0 || blockIdx.y != 0 || blockIdx.z != 0) return;
-  if (a.n_units == 0) {
-    if (threadIdx.x == 0) y[0] = 0.0f;
+  const uint32_t lane = threadIdx.x, nb = a.n_units;
+  if (nb == 0) {
+    if (lane == 0) y[0] = 0.0f;
     return;
   }
-  q4_0_matvec_body<1, 1>(q, x, y, 1u, a.n_units, kRefTileB, 0u, lds);
+  const uint32_t i = lane >> 2, t = lane & 3u;
+  auto load = [&](Ref0Iter &S, uint32_t it) { // past the last block: the last one again
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t blk = min(it * 64u + 16u * (uint32_t)u + i, nb - 1u);
+      const uint8_t *b = q + (size_t)blk * kQ4_0BlockBytes;
+      S.d[u] = *reinterpret_cast<const uint16_t *>(b);
+      S.qv[u] = *reinterpret_cast<const axh_u32u *>(b + 2u + 4u * t);
+      const float4 *xp = reinterpret_cast<const float4 *>(x + (size_t)blk * 32u) + t;
+      S.xl[u] = xp[0];
+      S.xh[u] = xp[4];
+    }
+  };
+  Ref0Iter S[kRef0Ahead];
+#pragma unroll
+  for (int p = 0; p < kRef0Ahead; ++p) load(S[p], (uint32_t)p);
+  __builtin_amdgcn_sched_barrier(0);
+  const uint32_t n_it = (nb + 63u) >> 6;
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (uint32_t it0 = 0; it0 < n_it; it0 += kRef0Ahead) {
+#pragma unroll
+    for (int p = 0; p < kRef0Ahead; ++p) {
+      const uint32_t it = it0 + (uint32_t)p;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float4 l = S[p].xl[u], h = S[p].xh[u];
+        float alo = 0.0f, ahi = 0.0f;
+        q4k_dword(S[p].qv[u], l, h, alo, ahi);
+        const float xs = ((l.x + l.y) + (l.z + l.w)) + ((h.x + h.y) + (h.z + h.w));
+        const float dot = __builtin_fmaf(16777216.0f, alo, 1048576.0f * ahi);
+        // a repeated last block adds +0 (masked bits: no branch per block)
+        const uint32_t m = it * 64u + 16u * (uint32_t)u + i < nb ? 0xFFFFFFFFu : 0u;
+        const uint32_t v = __builtin_bit_cast(uint32_t, __builtin_fmaf(-8.0f, xs, dot)) & m;
+        acc[u] = __builtin_fmaf(f16_to_f32(S[p].d[u] & m), __builtin_bit_cast(float, v), acc[u]);
+      }
+      __builtin_amdgcn_sched_barrier(0); // the loads stay ahead of the next compute
+      load(S[p], it + kRef0Ahead);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  const float r = wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+  if (lane == 0) y[0] = r;
 }
 
 // ===========================================================================
