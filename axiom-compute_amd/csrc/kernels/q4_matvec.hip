@@ -2717,6 +2717,27 @@ extern "C" __global__ void __launch_bounds__(256)
   }
 }
 
+// Copies between a dispatch's pinned staging buffer and its device buffers:
+// segment blockIdx.y of the table (which lies in the staging buffer itself),
+// 16 bytes per thread and step.  One launch moves every binding; the copy
+// engine took a submission of 8-15 us of host time per binding.  src and dst
+// are 16-byte aligned; the last bytes % 16 go one by one.
+struct CopySegment {
+  const uint8_t *src;
+  uint8_t *dst;
+  uint64_t bytes;
+};
+extern "C" __global__ void __launch_bounds__(256)
+    axh_copy_segments(const CopySegment *__restrict__ table, AXH_COUNT_ARGS) { AXH_COUNT_UNPACK;
+  if (blockIdx.y >= a.n_units) return;
+  const CopySegment s = table[blockIdx.y];
+  const uint64_t n16 = s.bytes >> 4;
+  for (uint64_t i = blockIdx.x * 256u + threadIdx.x; i < n16; i += gridDim.x * 256u)
+    reinterpret_cast<u32x4_t *>(s.dst)[i] = reinterpret_cast<const u32x4_t *>(s.src)[i];
+  const uint64_t tail = (n16 << 4) + threadIdx.x;
+  if (blockIdx.x == 0 && tail < s.bytes) s.dst[tail] = s.src[tail];
+}
+
 // Measurement helpers for the floor that one launch per call puts under a
 // matvec (no counterpart in the reference).  axh_read_floor streams
 // a.n_units 16-byte pieces of q with the matvec's launch shape (one 8-wave

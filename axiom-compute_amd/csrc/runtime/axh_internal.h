@@ -44,6 +44,9 @@ struct Core {
   // Staging buffers whose copy outlived a fence timeout (freed at teardown).
   std::vector<void *> retired_staging;
 
+  std::mutex event_mu;
+  std::vector<hipEvent_t> idle_events; // kept between completion waits
+
   std::mutex cache_mu; // guards modules and kernels
   std::unordered_map<uint64_t, LoadedModule> modules;
   std::unordered_map<uint64_t, axh_kernel *> kernels; // non-owning
@@ -71,6 +74,8 @@ struct axh_kernel {
   std::mutex mu;              // serialises dispatch_handle on this handle
   std::vector<void *> pool;   // per-binding device buffers
   std::vector<size_t> pool_bytes;
+  void *staging = nullptr; // pinned host memory of dispatch_handle (at most 32 MiB)
+  size_t staging_bytes = 0;
 };
 
 struct axh_context {

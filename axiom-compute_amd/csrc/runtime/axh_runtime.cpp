@@ -51,6 +51,7 @@ Core::~Core() {
   if (stream) hipStreamSynchronize(stream); // retired staging buffers may still be in use
   if (staging) hipHostFree(staging);
   for (void *p : retired_staging) hipHostFree(p);
+  for (hipEvent_t ev : idle_events) hipEventDestroy(ev);
   if (stream) hipStreamDestroy(stream);
 }
 
@@ -68,11 +69,26 @@ static uint64_t round_up_pow2(uint64_t v) {
 
 // Waits for all work queued on `stream` so far, polling an event so the wait
 // is bounded by the context's fence timeout (reference: vkWaitForFences with
-// AXC_FENCE_TIMEOUT_MS, kernel_handle.rs:672-686).
+// AXC_FENCE_TIMEOUT_MS, kernel_handle.rs:672-686).  The first kSpinUs are
+// polled without sleeping: a 20 us sleep takes 70-80 us with the default timer
+// slack, more than most waits last.  Events are kept for the next wait.
+static constexpr auto kSpinUs = std::chrono::microseconds(500);
+static constexpr size_t kMaxIdleEvents = 16;
+
 static axh_status wait_stream(Core &core, hipStream_t stream) {
-  hipEvent_t ev;
-  hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-  if (e != hipSuccess) return fail(AXH_ERR_QUEUE_SUBMIT, hip_msg("hipEventCreate", e));
+  hipEvent_t ev = nullptr;
+  {
+    std::lock_guard<std::mutex> lk(core.event_mu);
+    if (!core.idle_events.empty()) {
+      ev = core.idle_events.back();
+      core.idle_events.pop_back();
+    }
+  }
+  hipError_t e = hipSuccess;
+  if (!ev) {
+    e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess) return fail(AXH_ERR_QUEUE_SUBMIT, hip_msg("hipEventCreate", e));
+  }
   e = hipEventRecord(ev, stream);
   if (e != hipSuccess) {
     hipEventDestroy(ev);
@@ -80,7 +96,6 @@ static axh_status wait_stream(Core &core, hipStream_t stream) {
   }
   const auto t0 = std::chrono::steady_clock::now();
   const auto limit = std::chrono::milliseconds(core.fence_timeout_ms);
-  int spins = 0;
   for (;;) {
     e = hipEventQuery(ev);
     if (e == hipSuccess) break;
@@ -88,15 +103,20 @@ static axh_status wait_stream(Core &core, hipStream_t stream) {
       hipEventDestroy(ev);
       return fail(AXH_ERR_QUEUE_SUBMIT, hip_msg("hipEventQuery", e));
     }
-    if (std::chrono::steady_clock::now() - t0 > limit) {
+    const auto waited = std::chrono::steady_clock::now() - t0;
+    if (waited > limit) {
       hipEventDestroy(ev);
       return fail(AXH_ERR_FENCE_TIMEOUT,
                   "completion wait timed out after " +
                       std::to_string(core.fence_timeout_ms * 1000000ull) + " ns");
     }
-    if (++spins > 64) std::this_thread::sleep_for(std::chrono::microseconds(20));
+    if (waited > kSpinUs) std::this_thread::sleep_for(std::chrono::microseconds(20));
   }
-  hipEventDestroy(ev);
+  std::lock_guard<std::mutex> lk(core.event_mu);
+  if (core.idle_events.size() < kMaxIdleEvents)
+    core.idle_events.push_back(ev);
+  else
+    hipEventDestroy(ev);
   return AXH_OK;
 }
 
@@ -479,6 +499,7 @@ void axh_kernel_release(axh_kernel *k) {
     hipSetDevice(core->device);
     for (void *p : k->pool)
       if (p) hipFree(p);
+    if (k->staging) hipHostFree(k->staging);
     release_module(*core, k->module_hash);
   }
   delete k; // the last holder of `core` may free the device state here
@@ -489,6 +510,111 @@ uint64_t axh_kernel_cache_key(const axh_kernel *k) { return k ? k->key : 0; }
 uint64_t axh_kernel_pool_bytes(const axh_kernel *k, uint32_t binding) {
   if (!k || binding >= k->pool_bytes.size()) return 0;
   return k->pool_bytes[binding];
+}
+
+// A binding's share of a handle's staging buffer (256-byte aligned).
+static size_t staged_size(size_t bytes) {
+  return bytes > kStagingChunk ? kStagingChunk + 1 : (bytes + 255u) & ~size_t(255);
+}
+
+// axh_copy_segments' table entry (q4_matvec.hip).
+struct CopySegment {
+  const void *src;
+  void *dst;
+  uint64_t bytes;
+};
+// Bindings up to this size are copied by one kernel launch for all of them,
+// larger ones by the copy engine.
+static constexpr size_t kKernelCopyBytes = size_t(2) << 20;
+static constexpr uint32_t kCopyWgs = 64; // workgroups per segment
+
+// dispatch_handle's device work through the handle's staging buffer; k->mu is
+// held and the pool is sized.  The buffer holds the two segment tables, the
+// inputs and the outputs (`packed` bytes).
+static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
+                                  const void *const *inputs, const size_t *input_sizes,
+                                  const size_t *output_sizes, void *const *outputs, const void *pc,
+                                  size_t pc_bytes, size_t packed) {
+  Core &core = *ctx->core;
+  const size_t n = k->access.size();
+  axh_kernel *copy = nullptr;
+  axh_status s = builtin_kernel(ctx, "axh_copy_segments", 1, 4, 256, &copy);
+  if (s != AXH_OK) return s;
+  hipError_t e = hipSuccess;
+  if (k->staging_bytes < packed) {
+    if (k->staging) hipHostFree(k->staging);
+    k->staging = nullptr;
+    k->staging_bytes = 0;
+    const size_t want = round_up_pow2(packed);
+    e = hipHostMalloc(&k->staging, want, hipHostMallocDefault);
+    if (e != hipSuccess) return fail(AXH_ERR_MEMORY_MAP, hip_msg("hipHostMalloc", e));
+    k->staging_bytes = want;
+  }
+  // After an error copies may still be queued on the staging buffer: it is
+  // freed with the core, and the next dispatch takes a fresh one.
+  auto retire = [&](axh_status st) {
+    std::lock_guard<std::mutex> lk(core.staging_mu);
+    if (k->staging) core.retired_staging.push_back(k->staging);
+    k->staging = nullptr;
+    k->staging_bytes = 0;
+    return st;
+  };
+  auto copy_launch = [&](CopySegment *table, uint32_t segs, size_t largest) {
+    if (segs == 0) return AXH_OK;
+    const size_t wgs = (largest + 4095) / 4096; // 16 bytes per thread of a workgroup
+    const uint32_t grid[3] = {(uint32_t)(wgs < 1 ? 1 : wgs > kCopyWgs ? kCopyWgs : wgs), segs, 1};
+    void *bufs[1] = {table};
+    return launch_raw(copy, grid, bufs, 1, &segs, sizeof(segs), 0, core.stream);
+  };
+  CopySegment *tin = static_cast<CopySegment *>(k->staging), *tout = tin + n;
+  uint8_t *at = static_cast<uint8_t *>(k->staging) + staged_size(2 * n * sizeof(CopySegment));
+  uint32_t segs = 0;
+  size_t largest = 0;
+  for (size_t i = 0; i < n; ++i) {
+    if (input_sizes[i] == 0) continue;
+    std::memcpy(at, inputs[i], input_sizes[i]);
+    if (input_sizes[i] <= kKernelCopyBytes) {
+      tin[segs++] = CopySegment{at, k->pool[i], input_sizes[i]};
+      if (input_sizes[i] > largest) largest = input_sizes[i];
+    } else {
+      e = hipMemcpyAsync(k->pool[i], at, input_sizes[i], hipMemcpyHostToDevice, core.stream);
+      if (e != hipSuccess)
+        return retire(fail(AXH_ERR_STAGING_COPY, "binding #" + std::to_string(i) +
+                                                     " (HostToDevice): " +
+                                                     hip_msg("hipMemcpyAsync", e)));
+    }
+    at += staged_size(input_sizes[i]);
+  }
+  s = copy_launch(tin, segs, largest);
+  if (s != AXH_OK) return retire(s);
+  s = launch_raw(k, workgroups, k->pool.data(), n, pc, pc_bytes, 0, core.stream);
+  if (s != AXH_OK) return retire(s);
+  const uint8_t *out = at;
+  segs = 0;
+  largest = 0;
+  for (size_t i = 0; i < n; ++i) {
+    if (output_sizes[i] == 0) continue;
+    if (output_sizes[i] <= kKernelCopyBytes) {
+      tout[segs++] = CopySegment{k->pool[i], at, output_sizes[i]};
+      if (output_sizes[i] > largest) largest = output_sizes[i];
+    } else {
+      e = hipMemcpyAsync(at, k->pool[i], output_sizes[i], hipMemcpyDeviceToHost, core.stream);
+      if (e != hipSuccess)
+        return retire(fail(AXH_ERR_READBACK, "readback of binding #" + std::to_string(i) +
+                                                 " failed: " + hip_msg("hipMemcpyAsync", e)));
+    }
+    at += staged_size(output_sizes[i]);
+  }
+  s = copy_launch(tout, segs, largest);
+  if (s != AXH_OK) return retire(s);
+  s = wait_stream(core, core.stream);
+  if (s != AXH_OK) return retire(s);
+  for (size_t i = 0; i < n; ++i) {
+    if (output_sizes[i] == 0) continue;
+    std::memcpy(outputs[i], out, output_sizes[i]);
+    out += staged_size(output_sizes[i]);
+  }
+  return AXH_OK;
 }
 
 axh_status axh_dispatch_handle(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
@@ -540,6 +666,21 @@ axh_status axh_dispatch_handle(axh_context *ctx, axh_kernel *k, const uint32_t w
                                                  hip_msg("hipMalloc", e));
     k->pool[i] = p;
     k->pool_bytes[i] = sz;
+  }
+  // Requests up to kStagingChunk bytes go through the handle's own pinned
+  // buffer, inputs and outputs side by side: the copies and the launch are
+  // queued behind each other and waited for once.  Larger ones stage and wait
+  // for each binding by itself.
+  size_t packed = staged_size(2 * n * sizeof(CopySegment));
+  for (size_t i = 0; i < n; ++i) {
+    packed += staged_size(input_sizes[i]);
+    packed += staged_size(output_sizes[i]);
+    if (packed > kStagingChunk) break;
+  }
+  if (packed <= kStagingChunk) {
+    s = dispatch_packed(ctx, k, workgroups, inputs, input_sizes, output_sizes, outputs, pc,
+                        pc_bytes, packed);
+    return s == AXH_OK ? ok() : s;
   }
   for (size_t i = 0; i < n; ++i) {
     if (input_sizes[i] == 0) continue;

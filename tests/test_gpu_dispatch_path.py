@@ -47,3 +47,23 @@ def test_q4_0_single_output_iterations(ctx, axc, n):
     yf, ad = O.q4_0_matvec_f64(q, x, 1, n)
     rep = O.matvec_tolerance_report(y, O.q4_0_matvec(q, x, 1, n), yf, ad, n * 32, 1e-3)
     assert rep["ok"], rep
+
+
+# f16 words whose binding sizes lie around 16-byte pieces, one 4 KiB workgroup,
+# the largest size copied by the kernel (2 MiB: 2 n and 4 n bytes), and the
+# 32 MiB of one staged request (8 n bytes in all).
+@pytest.mark.parametrize("n", [1, 3, 7, 8, 9, 1023, 1024, 1025, 2048, (1 << 19) - 1, 1 << 19,
+                               (1 << 19) + 1, 1 << 20, (1 << 20) + 3, (1 << 22) - 200, 1 << 22])
+def test_dispatch_copies(ctx, axc, n):
+    """Both directions of every binding: h goes up and comes back, f = widen(h)."""
+    print(f"dispatch copies {n}", flush=True)
+    h = np.random.default_rng(n).integers(0, 0x7C00, n).astype(np.uint16)
+    k = ctx.prepare_kernel(axc.builtin_code_object(), _plan(axc, 2, 4, 256), 4, "axh_f16_widen")
+    for _ in range(2):  # the second one reuses the handle's staging buffer
+        out = ctx.dispatch_handle(k, ((n + 255) // 256, 1, 1), [h.tobytes(), b""],
+                                  [2 * n, 4 * n], struct.pack("<I", n))
+        assert out[0] == h.tobytes()
+        assert np.array_equal(np.frombuffer(out[1], np.float32),
+                              h.view(np.float16).astype(np.float32))
+        h = h[::-1].copy()
+    k.release()
