@@ -12,19 +12,22 @@
 // common_helpers.rs:437-454) and then rounded once to f16 (RN_f16(w32)).
 // f16 x f16 products are exact in the f32 accumulators of the MFMA.
 //
-// Four kernel kinds; the runtime picks one by the grid each would launch
+// Five kernel kinds; the runtime picks one by the grid each would launch
 // (the others stay reachable as strategy variants):
 //   * streaming rows (axh_q4k_matmul_sr_..., kind 7; K <= 4096): persistent,
 //     K split across the waves, X fragments kept in VGPRs, weights streamed
 //     like the matvec; see q4k_matmul_sr;
+//   * long rows (axh_q4k_matmul_lk_..., kind 9): 16- or 32-row tiles, K split
+//     across 8 waves, X in chunks through an LDS ring; see q4k_matmul_lk;
 //   * K-split (axh_q4k_matmul_ks_..., kind 3): the waves of a workgroup share
 //     one 32-row tile and split K, summing in LDS; see q4k_matmul_ks;
-//   * K-split tile (axh_q4k_matmul_kx_..., kind 5): the waves of a workgroup
-//     split K, each streaming raw weight bytes and X through a private LDS
-//     ring filled by coalesced direct-to-LDS loads; see q4k_matmul_kx;
-//   * 32 x 32 tiles (axh_q4k_matmul_rm_..., kind 8): waves of 32-row MFMA
-//     tiles over 128 columns, X and weights through a 4-deep LDS ring; see
-//     q4k_matmul_rm.
+//   * K-split tile (axh_q4k_matmul_kx_..., kind 5) and 32 x 32 tiles
+//     (axh_q4k_matmul_rm_..., kind 8): the main forms of both, from 64 rows x
+//     32 columns to 256 x 128, share one body, 8 waves of 32-row MFMA tiles
+//     over whole superblocks; see q4k_matmul_wk.  The other forms, and those
+//     for rows of few superblocks (_short), keep the bodies of q4k_matmul_kx
+//     (each wave streams 64-wide chunks through a private LDS ring) and
+//     q4k_matmul_rm (waves of 32-row tiles, a shared 4-deep ring).
 #include "q4_common.h"
 
 using namespace axh;
@@ -721,7 +724,8 @@ __device__ __forceinline__ void q4k_matmul_lk(const uint8_t *__restrict__ q,
 }
 
 // ---------------------------------------------------------------------------
-// 32 x 32 tiles with wide waves (kind 8, axh_q4k_matmul_rm_w{W}_r{RT}_p4): a
+// 32 x 32 tiles with wide waves (kind 8's forms of 64 rows per wave, and of few
+// superblocks; axh_q4k_matmul_rm_w{W}_r{RT}_p4): a
 // workgroup of W waves owns 32 * RT * W rows x 128 columns of Y; wave w owns
 // 32 * RT rows (RT 32-row MFMA tiles) x 128 columns (four 32-column tiles) and
 // walks all of K in 64-wide steps (one chunk of a superblock) with
@@ -957,6 +961,403 @@ __device__ __forceinline__ void q4k_matmul_rm(const uint8_t *__restrict__ q,
                    n_rows, v);
       }
     }
+}
+
+// ---------------------------------------------------------------------------
+// Wide K steps (the main kernels of kinds 5 and 8): 8 waves, each a 32-row
+// by 32 * CT-column tile of v_mfma_f32_32x32x16_f16.  KQ waves split K (wave w:
+// superblocks KQ c + w % KQ), the others take further rows, so a workgroup
+// owns 256 / KQ rows by 32 * CT columns.
+// A step is one 64-wide chunk of the superblock each wave is at; A fragments
+// and X fragments as in q4k_matmul_rm, prepared during the previous step's
+// MFMAs in a fixed order (one MFMA, then its share of the next step's
+// dequantisation, sched_barrier between them).
+// X goes through a ring of kRing LDS buffers (KQ groups x C columns x 128
+// bytes) kAhead steps ahead.  A wave's weights are its own: the whole 144
+// bytes of its 32 rows of one superblock go through LDS (a chunk's 48 bytes per
+// row and step, header included, as q4k_matmul_rm reads them, are a third more
+// loads) and to registers a superblock ahead; the next superblock's follow
+// into the same LDS as soon as they are read.  Past 16 KiB of X per step the
+// headers are loaded straight to registers, which leaves LDS for a further X
+// buffer.  The last nsb % KQ superblocks are dealt out by chunks and come
+// first, their weights straight to registers: dealt out whole they would leave
+// groups idle for a round and make the others' sums longer (14336 x 1536 x 128
+// error 1.40e-7 against 1.33e-7 in 64 bits, now 1.32e-7).
+//
+// What bounds it: the vector unit's issue slots.  A 32x32x16 MFMA is 35 cycles
+// of the matrix core and its 5 VALU instructions of dequantisation (at 128
+// columns; 20 at 32) take 4 to 5 cycles each beside it, for two waves per
+// SIMD; at 512 columns the card's power adds to that (the clock falls from 2.4
+// to 1.8 GHz, and a copy of the kernel without its waits takes as long).
+// Measured against the bodies it replaced (four waves, 64-wide chunks dealt
+// out to K groups or whole rows, headers decoded per chunk), same tiles, us:
+// 14336 x 4096 x 512 75.4 -> 68.4, x 256 42 -> 36.5, x 64 20.6 -> 18.2, x 128
+// 27.4 -> 26.4; 28672 x 14336 x 256 265 -> 217; 4096 x 14336 x 128 44.5 -> 36;
+// 5000 x 11008 x 77 36.4 -> 29.1 with the f32 cast.  Errors against 64 bits
+// are the same, or lower where K is split in more groups than before.
+// ---------------------------------------------------------------------------
+template <int KQ, int CT>
+__device__ __forceinline__ void q4k_matmul_wk(const uint8_t *__restrict__ q,
+                                              const uint16_t *__restrict__ x,
+                                              float *__restrict__ y, const MatmulArgs a,
+                                              f32x4_t *lds) {
+  static_assert(KQ == 1 || KQ == 2 || KQ == 4 || KQ == 8, "K groups of the 8 waves");
+  static_assert(KQ * CT == 4 || KQ * CT == 8 || KQ * CT == 16, "16, 32 or 64 KiB of X per step");
+  // X(j + kAhead) is issued in step j.  A buffer is free one step after its
+  // fragments were read; with two buffers (kEarly) in the step right after,
+  // once every wave's reads have returned.
+  constexpr bool kEarly = KQ * CT == 16;
+  constexpr int NW = 8, kRing = KQ * CT == 4 ? 6 : KQ * CT == 8 ? 4 : 2;
+  constexpr int kAhead = kEarly ? kRing : kRing - 1;
+  constexpr int kSlots = 4 * CT, kTasks = 21;
+  constexpr uint32_t C = 32u * CT;
+  constexpr uint32_t kXSlot = KQ * C * 8u;   // f32x4 of an X buffer
+  constexpr uint32_t kWOff = kRing * kXSlot; // the waves' weights follow
+  constexpr bool kHdrLds = KQ * CT == 4;      // headers through LDS, or straight to registers
+  constexpr uint32_t kPieces = kHdrLds ? 9u : 8u; // 16-byte pieces of a row in LDS
+  constexpr uint32_t kWSlot = 32u * kPieces;  // f32x4 of a wave's rows
+  constexpr int kXI = KQ * C / 8 / NW;       // X instructions per wave per step
+  constexpr int kWI = kHdrLds ? 5 : 4;       // weight instructions per superblock
+  constexpr int kHI = kHdrLds ? 0 : 1;       // header loads per superblock
+  constexpr uint32_t kFar = 0xFFF00000u;     // reads zeros, with room for SGPR offsets
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t kq = wave % KQ, rg = wave / KQ;
+  const uint32_t r = lane & 31u, h = lane >> 5;
+  const uint32_t n_rows = a.n_rows, nsb = a.sb_per_row, batch = a.batch;
+  const uint32_t K = nsb * 256u;
+  // Steps: n_first over the last nsb % KQ superblocks (step i, K group g:
+  // chunk KQ i + g of them, so that the groups stay even), then n_steps over
+  // whole rounds of KQ superblocks.
+  constexpr int kFirst = KQ == 1 ? 0 : KQ == 8 ? 4 : 4 - 4 / KQ; // at most
+  const uint32_t nsb_main = nsb / KQ * KQ;
+  const uint32_t n_steps = 4u * (nsb_main / KQ);
+  const uint32_t n_first = (4u * (nsb - nsb_main) + KQ - 1u) / KQ;
+  const uint32_t row_bytes = nsb * (uint32_t)kQ4kSbBytes;
+  const uint32_t m0 = blockIdx.x * (256u / KQ) + 32u * rg, n0 = blockIdx.y * C;
+
+  // X load role: instruction i = wave + 8 u of a step covers virtual columns
+  // v = 8 i .. 8 i + 7 (K group v / C, column v % C), lane l piece (l & 7) ^
+  // ((v >> 1) & 7) of column 8 i + l / 8.
+  uint32_t xv0[kXI];
+#pragma unroll
+  for (int u = 0; u < kXI; ++u) {
+    const uint32_t v = 8u * (wave + NW * (uint32_t)u) + (lane >> 3);
+    const uint32_t p = (lane & 7u) ^ ((v >> 1) & 7u), b = n0 + (v & (C - 1u));
+    xv0[u] = b < batch ? (b * K + 8u * p) * 2u : kFar;
+  }
+  // Weight load role: LDS piece P = 64 m + lane is piece P % kPieces of the
+  // wave's row P / kPieces: the row's 9 pieces in order (an odd stride: no
+  // bank conflicts), or its 8 qs pieces, number p in place p ^ ((row >> 1) & 7).
+  uint32_t wv0[kWI];
+#pragma unroll
+  for (int m = 0; m < kWI; ++m) {
+    const uint32_t P = 64u * (uint32_t)m + lane, rr = P / kPieces, row = m0 + rr;
+    const uint32_t p = kHdrLds ? P - 9u * rr : 1u + ((P & 7u) ^ ((rr >> 1) & 7u));
+    wv0[m] = rr < 32u && row < n_rows ? row * row_bytes + 16u * p : kFar;
+  }
+  const uint32_t hv0 = m0 + r < n_rows ? (m0 + r) * row_bytes : kFar;
+  // Past the last superblock the loads go through an empty resource.
+  auto issue_x_at = [&](uint32_t sb, uint32_t chunk, bool real, uint32_t slot, int u) {
+    const uint32_t i = wave + NW * (uint32_t)u;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(x, real ? batch * K * 2u : 0u),
+                                             (lds_void_t *)(lds + slot * kXSlot + i * 64u), 16,
+                                             xv0[u], sb * 512u + 128u * chunk, 0, 0);
+  };
+  auto issue_x = [&](uint32_t j, uint32_t slot, int u) { // step j of the whole rounds
+    const uint32_t sb = KQ * (j >> 2) + 8u * (wave + NW * (uint32_t)u) / C;
+    issue_x_at(sb, j & 3u, sb < nsb_main, slot, u);
+  };
+  auto issue_x_first = [&](uint32_t i, uint32_t slot, int u) { // step i of all
+    if (i >= n_first) {
+      issue_x(i - n_first, slot, u);
+    } else {
+      const uint32_t f = KQ * i + 8u * (wave + NW * (uint32_t)u) / C, sb = nsb_main + (f >> 2);
+      issue_x_at(sb, f & 3u, sb < nsb, slot, u);
+    }
+  };
+  f32x4_t *const wb = lds + kWOff + wave * kWSlot;
+  auto issue_w = [&](uint32_t c, int m) { // chunk c's superblock of this wave
+    const uint32_t sb = KQ * c + kq;
+    if (64u * (uint32_t)m + 64u <= kWSlot || lane < (kWSlot & 63u))
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(q, sb < nsb_main ? n_rows * row_bytes : 0u),
+                                               (lds_void_t *)(wb + 64 * m), 16, wv0[m], sb * 144u,
+                                               0, 0);
+  };
+  // The superblock in registers: header and this lane's half of each chunk.
+  uint4 hd, qv[4], hdn, qvn[4];
+  auto load_h = [&](uint32_t c) {
+    const uint32_t sb = KQ * c + kq;
+    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(
+        rsrc(q, sb < nsb_main ? n_rows * row_bytes : 0u), (int)hv0, (int)(sb * 144u), 0);
+    hdn = make_uint4(v.x, v.y, v.z, v.w);
+  };
+  auto read_w = [&]() { // a header in LDS comes last: once it is here, all are
+#pragma unroll
+    for (uint32_t n = 0; n < 4u; ++n)
+      qvn[n] = __builtin_bit_cast(
+          uint4, wb[kHdrLds ? 9u * r + 1u + 2u * n + h : 8u * r + ((2u * n + h) ^ ((r >> 1) & 7u))]);
+    if constexpr (kHdrLds) hdn = __builtin_bit_cast(uint4, wb[9u * r]);
+  };
+  auto take_w = [&]() {
+    hd = hdn;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) qv[n] = qvn[n];
+  };
+  // X fragment (k-step s, column tile t): piece (s & 1) + 2 h + 4 (s >> 1) of
+  // virtual column C kq + 32 t + r.
+  uint32_t xl[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const uint32_t p = ((uint32_t)s & 1u) + 2u * h + 4u * ((uint32_t)s >> 1);
+    xl[s] = 8u * (C * kq + r) + (p ^ ((r >> 1) & 7u));
+  }
+  f32x16_t acc[CT];
+#pragma unroll
+  for (int t = 0; t < CT; ++t) acc[t] = (f32x16_t){};
+  half8_t af[2][4], bf[4][CT];
+  uint32_t frag[4][4];
+
+  // Task T of step j + 1's dequantisation (chunk cn of hd / qv): the
+  // superblock's 16 scales and mins as bytes (first chunk only: 14 VALU per
+  // superblock instead of 10 per chunk), the chunk's four factors, then 8 half
+  // dwords u (dword u / 2, low or high nibbles) of two tasks each: masks and
+  // two FMAs, then two FMAs and the packing of half dword u - 1.
+  float d24, d20, dm, d1s, d2s, m1, m2, f[2][4];
+  uint32_t sclo, schi, mlo, mhi, lb, hb;
+  auto pack_half = [&](int u) {
+    const int dw = u >> 1, hi = u & 1;
+    uint32_t &a0 = frag[2 * hi + (dw >> 1)][2 * (dw & 1)];
+    uint32_t &a1 = frag[2 * hi + (dw >> 1)][2 * (dw & 1) + 1];
+    a0 = pack_f16(f[u & 1][0], f[u & 1][1]);
+    a1 = pack_f16(f[u & 1][2], f[u & 1][3]);
+    asm volatile("" ::"v"(a0), "v"(a1)); // computed here, not sunk to the step's end
+  };
+  auto task = [&](int k, int cn) {
+    if (k == 0) {
+      if (cn != 0) return;
+      const float d = f16_to_f32(hd.x & 0xFFFFu);
+      dm = f16_to_f32(hd.x >> 16);
+      d24 = d * 16777216.0f;
+      d20 = d * 1048576.0f;
+      sclo = hd.y & 0x3F3F3F3Fu;
+      mlo = hd.z & 0x3F3F3F3Fu;
+      asm volatile("" ::"v"(dm), "v"(d24), "v"(d20), "v"(sclo), "v"(mlo));
+    } else if (k == 1) {
+      if (cn != 0) return;
+      schi = (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u);
+      mhi = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
+      asm volatile("" ::"v"(schi), "v"(mhi));
+    } else if (k < 4) { // sub-block 2 cn + k - 2: byte 2 cn + k - 2 of eight
+      const uint32_t sh = 8u * (uint32_t)(2 * (cn & 1) + k - 2);
+      const float sc = (float)(((cn < 2 ? sclo : schi) >> sh) & 0xFFu);
+      const float mm = (float)(((cn < 2 ? mlo : mhi) >> sh) & 0xFFu);
+      if (k == 2) {
+        d1s = d24 * sc;
+        m1 = dm * mm;
+        asm volatile("" ::"v"(d1s), "v"(m1));
+      } else {
+        d2s = d20 * sc;
+        m2 = dm * mm;
+        asm volatile("" ::"v"(d2s), "v"(m2));
+      }
+    } else if (k < 20) {
+      const int t = k - 4, u = t >> 1, dw = u >> 1, hi = u & 1;
+      const uint4 qc = qv[cn];
+      const uint32_t w = dw == 0 ? qc.x : dw == 1 ? qc.y : dw == 2 ? qc.z : qc.w;
+      const float ds = hi ? d2s : d1s, m = hi ? m2 : m1;
+      float *fu = f[u & 1];
+      if ((t & 1) == 0) {
+        lb = w & (hi ? 0x00F000F0u : 0x000F000Fu);
+        hb = (w >> 8) & (hi ? 0x00F000F0u : 0x000F000Fu);
+        fu[0] = __builtin_fmaf(lo_half_f16(lb), ds, -m);
+        fu[1] = __builtin_fmaf(lo_half_f16(hb), ds, -m);
+        asm volatile("" ::"v"(fu[0]), "v"(fu[1]));
+      } else {
+        fu[2] = __builtin_fmaf(hi_half_f16(lb), ds, -m);
+        fu[3] = __builtin_fmaf(hi_half_f16(hb), ds, -m);
+        asm volatile("" ::"v"(fu[2]), "v"(fu[3]));
+        if (u > 0) pack_half(u - 1);
+      }
+    } else {
+      pack_half(7);
+    }
+  };
+  auto take_frag = [&](int b) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      af[b][s] = __builtin_bit_cast(
+          half8_t, make_uint4(frag[s][0], frag[s][1], frag[s][2], frag[s][3]));
+  };
+
+  // Prologue: the first steps' weights straight to registers, the loads that
+  // steps before the first would have issued, the first steps; W(1) once W(0)
+  // is in registers.
+  uint4 hf[kFirst ? kFirst : 1], qf[kFirst ? kFirst : 1];
+#pragma unroll
+  for (int i = 0; i < kFirst; ++i) {
+    if ((uint32_t)i >= n_first) break;
+    const uint32_t f = KQ * (uint32_t)i + kq, sb = nsb_main + (f >> 2);
+    const __amdgpu_buffer_rsrc_t qr = rsrc(q, sb < nsb ? n_rows * row_bytes : 0u);
+    const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(qr, (int)hv0, (int)(sb * 144u), 0);
+    const u32x4_t w = __builtin_amdgcn_raw_buffer_load_b128(
+        qr, (int)(hv0 + 16u + 16u * h), (int)(sb * 144u + 32u * (f & 3u)), 0);
+    hf[i] = make_uint4(v.x, v.y, v.z, v.w);
+    qf[i] = make_uint4(w.x, w.y, w.z, w.w);
+  }
+  if constexpr (!kHdrLds) load_h(0u);
+#pragma unroll
+  for (int m = 0; m < kWI; ++m) issue_w(0u, m);
+#pragma unroll
+  for (uint32_t j = 0; j < (uint32_t)kAhead; ++j)
+#pragma unroll
+    for (int u = 0; u < kXI; ++u) issue_x_first(j, j, u);
+  // X(i), and at the end W(0), have landed when only kAhead - 1 steps of X
+  // came after them.
+#pragma unroll
+  for (int i = 0; i < kFirst; ++i) {
+    if ((uint32_t)i >= n_first) break;
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((kAhead - 1) * kXI) : "memory");
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int t = 0; t < CT; ++t)
+        bf[s][t] = __builtin_bit_cast(half8_t, lds[(i % kRing) * kXSlot + xl[s] + 256u * (uint32_t)t]);
+    if constexpr (kEarly) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int u = 0; u < kXI; ++u) issue_x_first(i + kAhead, (i + kAhead) % kRing, u);
+    const uint32_t ch = (KQ * (uint32_t)i + kq) & 3u, sh = 16u * (ch & 1u);
+    const uint32_t sc8 = ch < 2u ? hf[i].y & 0x3F3F3F3Fu
+                                 : (hf[i].w & 0x0F0F0F0Fu) | ((hf[i].y >> 2) & 0x30303030u);
+    const uint32_t mn8 = ch < 2u ? hf[i].z & 0x3F3F3F3Fu
+                                 : ((hf[i].w >> 4) & 0x0F0F0F0Fu) | ((hf[i].z >> 2) & 0x30303030u);
+    const float d0 = f16_to_f32(hf[i].x & 0xFFFFu), dm0 = f16_to_f32(hf[i].x >> 16);
+    const float s1 = (float)((sc8 >> sh) & 0xFFu), s2 = (float)((sc8 >> (sh + 8u)) & 0xFFu);
+    const float n1 = (float)((mn8 >> sh) & 0xFFu), n2 = (float)((mn8 >> (sh + 8u)) & 0xFFu);
+    const uint32_t qw[4] = {qf[i].x, qf[i].y, qf[i].z, qf[i].w};
+#pragma unroll
+    for (int dw = 0; dw < 4; ++dw) {
+      uint32_t *lo = &frag[dw >> 1][2 * (dw & 1)], *hi = &frag[2 + (dw >> 1)][2 * (dw & 1)];
+      dequant_dword(qw[dw], d0 * 16777216.0f * s1, dm0 * n1, d0 * 1048576.0f * s2, dm0 * n2, lo[0],
+                    lo[1], hi[0], hi[1]);
+    }
+    take_frag(0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int t = 0; t < CT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[0][s], bf[s][t], acc[t], 0, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((kAhead - 1) * kXI) : "memory");
+  read_w();
+  const uint32_t slot0 = n_first % (uint32_t)kRing;
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+      bf[s][t] = __builtin_bit_cast(half8_t, lds[slot0 * kXSlot + xl[s] + 256u * (uint32_t)t]);
+  take_w();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int m = 0; m < kWI; ++m) issue_w(1u, m);
+#pragma unroll
+  for (int T = 0; T < kTasks; ++T) task(T, 0);
+  take_frag(0);
+
+  // ring slots of X(j + 1) and X(j + kAhead)
+  uint32_t rd = (n_first + 1u) % (uint32_t)kRing, wr = (n_first + (uint32_t)kAhead) % (uint32_t)kRing;
+  auto step = [&](uint32_t jj, auto e_c) {
+    constexpr int e = decltype(e_c)::value; // jj % 4: the chunk
+    // Loads of a step: X(jj + kAhead); then at e = 3 the weights W(c + 2)
+    // of c = jj / 4, and at e = 0 the headers H(c + 1).  Own loads of
+    // X(jj + 1) have landed when only what came after them is in flight: the
+    // rest of step jj + 1 - kAhead and all of the steps since.  After the
+    // barrier every wave's are there, and X(jj - 1)'s buffer (X(jj)'s with
+    // kEarly: its reads are waited for) is free.
+    constexpr int kAfter = [] {
+      int n = 0;
+      for (int b = kAhead - 1; b >= 1; --b) { // step jj - b
+        const int eb = (e - b + 8) & 3;
+        n += (b < kAhead - 1 ? kXI : 0) + (eb == 3 ? kWI : eb == 0 ? kHI : 0);
+      }
+      return n;
+    }();
+    if constexpr (kEarly)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kAfter) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kAfter) : "memory");
+    const f32x4_t *bufn = lds + rd * kXSlot; // past the last step: read, never used
+    const uint32_t wrs = wr;
+    rd = rd + 1u == (uint32_t)kRing ? 0u : rd + 1u;
+    wr = wr + 1u == (uint32_t)kRing ? 0u : wr + 1u;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+      const int s = k / CT, t = k % CT;
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[e & 1][s], bf[s][t], acc[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = k; u < kXI; u += kSlots) issue_x(jj + (uint32_t)kAhead, wrs, u);
+      bf[s][t] = __builtin_bit_cast(half8_t, bufn[xl[s] + 256u * (uint32_t)t]);
+#pragma unroll
+      for (int T = k * kTasks / kSlots; T < (k + 1) * kTasks / kSlots; ++T) task(T, (e + 1) & 3);
+      if (!kHdrLds && e == 0 && k == kSlots - 1) load_h((jj >> 2) + 1u);
+      if (e == 3 && k == kSlots - 1) {
+        // the superblock now in registers leaves the buffer to the next one
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int m = 0; m < kWI; ++m) issue_w((jj >> 2) + 2u, m);
+      }
+      if (e == 2 && k == kSlots - (kSlots > 4 ? 2 : 1)) {
+        // own next weights: three steps' X and the headers came after them
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * kXI + kHI) : "memory");
+        read_w();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    take_frag((e & 1) ^ 1);
+    if (e == 2) take_w();
+  };
+  for (uint32_t j = 0; j < n_steps; j += 4) {
+    step(j, std::integral_constant<int, 0>{});
+    step(j + 1u, std::integral_constant<int, 1>{});
+    step(j + 2u, std::integral_constant<int, 2>{});
+    step(j + 3u, std::integral_constant<int, 3>{});
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // loads past the last step
+
+  auto store = [&](int t, int q4, f32x4_t v) {
+    const uint32_t b = n0 + 32u * (uint32_t)t + r;
+    if (b < batch)
+      store_col4(y + (size_t)b * n_rows, m0 + 8u * (uint32_t)q4 + 4u * h, n_rows, v);
+  };
+  auto quarter = [&](int t, int q4) {
+    return (f32x4_t){acc[t][4 * q4], acc[t][4 * q4 + 1], acc[t][4 * q4 + 2], acc[t][4 * q4 + 3]};
+  };
+  if constexpr (KQ == 1) {
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) store(t, q4, quarter(t, q4));
+  } else {
+    // Partial tiles of the K groups -> LDS, summed in K-group order
+    // (deterministic); wave kq of a row group takes every KQ-th quarter tile.
+    constexpr uint32_t kUnits = CT * 4;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+        lds[(wave * kUnits + (uint32_t)(t * 4 + q4)) * 64u + lane] = quarter(t, q4);
+    __syncthreads();
+    for (uint32_t unit = kq; unit < kUnits; unit += KQ) {
+      f32x4_t sum = lds[(rg * KQ * kUnits + unit) * 64u + lane];
+#pragma unroll
+      for (uint32_t k2 = 1; k2 < (uint32_t)KQ; ++k2)
+        sum += lds[((rg * KQ + k2) * kUnits + unit) * 64u + lane];
+      store((int)(unit >> 2), (int)(unit & 3u), sum);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1236,37 +1637,35 @@ AXH_Q4K_MATMUL_KS(8, 2, 1, 2, )
 AXH_Q4K_MATMUL_KS(8, 1, 1, 1, _r1)
 AXH_Q4K_MATMUL_KS(8, 1, 2, 1, _r1)
 
-#define AXH_Q4K_MATMUL_KX(RT, NT, KS, PF)                                                        \
+#define AXH_Q4K_MATMUL_KX(RT, NT, KS, PF, SUFFIX)                                                \
   extern "C" __global__ void __launch_bounds__(KS * 64)                                          \
-      axh_q4k_matmul_kx_r##RT##_n##NT##_k##KS##_p##PF(const uint8_t *__restrict__ q,             \
+      axh_q4k_matmul_kx_r##RT##_n##NT##_k##KS##_p##PF##SUFFIX(const uint8_t *__restrict__ q,     \
                                                       const uint16_t *__restrict__ x,            \
                                                       float *__restrict__ y, AXH_MATMUL_ARGS) { AXH_MATMUL_UNPACK; \
     extern __shared__ f32x4_t axh_red_dyn[];                                                     \
     q4k_matmul_kx<RT, NT, KS, PF>(q, x, y, a, axh_red_dyn);                                      \
   }
 
-AXH_Q4K_MATMUL_KX(4, 8, 4, 2)
-AXH_Q4K_MATMUL_KX(2, 8, 4, 2)
-AXH_Q4K_MATMUL_KX(4, 4, 4, 2)
-AXH_Q4K_MATMUL_KX(4, 4, 4, 3)
-AXH_Q4K_MATMUL_KX(8, 4, 4, 2)
-AXH_Q4K_MATMUL_KX(4, 2, 4, 2)
-AXH_Q4K_MATMUL_KX(4, 2, 4, 3)
-AXH_Q4K_MATMUL_KX(4, 1, 4, 3)
+AXH_Q4K_MATMUL_KX(2, 8, 4, 2, )
+AXH_Q4K_MATMUL_KX(4, 4, 4, 3, )
+AXH_Q4K_MATMUL_KX(8, 4, 4, 2, )
+AXH_Q4K_MATMUL_KX(4, 2, 4, 2, _short)
+AXH_Q4K_MATMUL_KX(4, 2, 4, 3, _short)
+AXH_Q4K_MATMUL_KX(4, 4, 4, 2, _short)
+AXH_Q4K_MATMUL_KX(4, 8, 4, 2, _short)
 
-#define AXH_Q4K_MATMUL_RM(W, RT)                                                                 \
+#define AXH_Q4K_MATMUL_RM(W, RT, SUFFIX)                                                         \
   extern "C" __global__ void __launch_bounds__(W * 64)                                           \
-      axh_q4k_matmul_rm_w##W##_r##RT##_p4(const uint8_t *__restrict__ q,                         \
+      axh_q4k_matmul_rm_w##W##_r##RT##_p4##SUFFIX(const uint8_t *__restrict__ q,                 \
                                           const uint16_t *__restrict__ x, float *__restrict__ y,  \
                                           AXH_MATMUL_ARGS) { AXH_MATMUL_UNPACK;                   \
     extern __shared__ f32x4_t axh_rm_dyn[];                                                      \
     q4k_matmul_rm<W, RT>(q, x, y, a, axh_rm_dyn);                                                \
   }
 
-AXH_Q4K_MATMUL_RM(4, 2)
-AXH_Q4K_MATMUL_RM(8, 1)
-AXH_Q4K_MATMUL_RM(4, 1)
-AXH_Q4K_MATMUL_RM(2, 2)
+AXH_Q4K_MATMUL_RM(4, 2, )
+AXH_Q4K_MATMUL_RM(2, 2, )
+AXH_Q4K_MATMUL_RM(4, 1, _short)
 
 #define AXH_Q4K_MATMUL_SR(NW, SPW, NC, XH, SUFFIX)                                               \
   extern "C" __global__ void __launch_bounds__(NW * 64)                                          \
@@ -1278,7 +1677,6 @@ AXH_Q4K_MATMUL_RM(2, 2)
   }
 
 AXH_Q4K_MATMUL_SR(8, 2, 1, false, )
-AXH_Q4K_MATMUL_SR(8, 2, 2, false, _n2)
 AXH_Q4K_MATMUL_SR(8, 2, 1, true, _h)
 
 #define AXH_Q4K_MATMUL_LK(XC, XD, WD, RT, SUFFIX)                                               \
@@ -1297,3 +1695,47 @@ AXH_Q4K_MATMUL_LK(16, 1, 3, 1, )
 AXH_Q4K_MATMUL_LK(8, 2, 2, 2, _r2)
 AXH_Q4K_MATMUL_LK(4, 2, 2, 1, )
 AXH_Q4K_MATMUL_LK(16, 1, 3, 2, _r2)
+
+#define AXH_Q4K_MATMUL_WK(KQ, CT, NAME)                                                         \
+  extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))   \
+      axh_q4k_matmul_##NAME(const uint8_t *__restrict__ q, const uint16_t *__restrict__ x,       \
+                            float *__restrict__ y, AXH_MATMUL_ARGS) {                            \
+    AXH_MATMUL_UNPACK;                                                                           \
+    extern __shared__ f32x4_t axh_wk_dyn[];                                                      \
+    q4k_matmul_wk<KQ, CT>(q, x, y, a, axh_wk_dyn);                                               \
+  }
+
+// 64 rows x 32, 64 or 128 columns with K in 4; 128 or 256 rows x 128 columns
+// with K in 2 or whole.  Their _short forms take rows of few superblocks.
+AXH_Q4K_MATMUL_WK(4, 1, kx_r4_n2_k4_p2)
+AXH_Q4K_MATMUL_WK(4, 1, kx_r4_n2_k4_p3)
+AXH_Q4K_MATMUL_WK(4, 2, kx_r4_n4_k4_p2)
+AXH_Q4K_MATMUL_WK(4, 4, kx_r4_n8_k4_p2)
+AXH_Q4K_MATMUL_WK(2, 4, rm_w4_r1_p4)
+AXH_Q4K_MATMUL_WK(1, 4, rm_w8_r1_p4)
+
+// Two kernels have a second body, 32 rows x 32 columns with K in 8, which the
+// host selects by shape (a.pad = 1, see matmul_launch_of): past one 16-row
+// block per workgroup (streaming rows) and past 16 columns (one-column-tile
+// K-split tiles, whose four waves let the other four end at once).
+extern "C" __global__ void __launch_bounds__(512)
+    axh_q4k_matmul_sr_w8_s2_n2(const uint8_t *__restrict__ q, const uint16_t *__restrict__ x,
+                               float *__restrict__ y, AXH_MATMUL_ARGS) {
+  AXH_MATMUL_UNPACK;
+  extern __shared__ f32x4_t axh_sr_dyn[];
+  if (a.pad != 0u)
+    q4k_matmul_wk<8, 1>(q, x, y, a, axh_sr_dyn);
+  else
+    q4k_matmul_sr<8, 2, 2, false>(q, x, y, a, axh_sr_dyn);
+}
+
+extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
+    axh_q4k_matmul_kx_r4_n1_k4_p3(const uint8_t *__restrict__ q, const uint16_t *__restrict__ x,
+                                  float *__restrict__ y, AXH_MATMUL_ARGS) {
+  AXH_MATMUL_UNPACK;
+  extern __shared__ f32x4_t axh_kx1_dyn[];
+  if (a.pad != 0u)
+    q4k_matmul_wk<8, 1>(q, x, y, a, axh_kx1_dyn);
+  else if (threadIdx.x < 256u)
+    q4k_matmul_kx<4, 1, 4, 3>(q, x, y, a, axh_kx1_dyn);
+}

@@ -1648,6 +1648,75 @@ constexpr uint64_t kMatmulCus = 256;
 // workgroups 21.5 us, 32 x 32 MFMA tiles in 64 workgroups 37.6).
 constexpr uint64_t kMatmulFill = 160;
 
+// Whether a kind 5 or 8 variant runs the wide-K-step body: its 8 waves split K
+// in 4 or 2, and rows too short for that (fewer than two rounds of 4
+// superblocks: 4096 rows x 128 columns, K = 1536 7.7 us with the narrow steps
+// against 8.6, 2048 9.2 against 8.9, 4096 15.2 against 13.3, 14080 43.8 against
+// 38.5; two rounds of 2: 12000 x 256 columns, K = 768 13.4 against 14.2, 1024
+// equal, 2304 27.4 against 24.9, 14080 135 against 111) go to the _short form
+// of the kernel.
+static bool matmul_wide(const MatmulVariant &v, uint32_t nsb) {
+  if (v.kind == 5) return v.rt == 4 && v.nt > 1 && !(v.nt == 4 && v.pf == 3) && nsb >= 8;
+  return v.kind == 8 && v.rt == 1 && (v.w == 8 || nsb >= 4);
+}
+static bool matmul_short(const MatmulVariant &v, uint32_t nsb) {
+  return !matmul_wide(v, nsb) && matmul_wide(v, UINT32_MAX);
+}
+
+// What a matmul variant launches for a shape: outputs per workgroup, threads,
+// LDS, and whether its kernel runs its second body.
+struct MatmulLaunch {
+  uint32_t rows, cols, threads, lds, second;
+};
+
+static MatmulLaunch matmul_launch_of(const MatmulVariant &v, uint32_t n_rows, uint32_t batch,
+                                     uint32_t nsb) {
+  const auto groups = [&](uint32_t rows_per_wg, uint32_t cols_per_wg) {
+    return (uint64_t)((n_rows + rows_per_wg - 1) / rows_per_wg) *
+           ((batch + cols_per_wg - 1) / cols_per_wg);
+  };
+  MatmulLaunch l{};
+  l.rows = v.kind == 8 ? 32u * v.rt * v.w : v.kind == 7 ? 16u : 16u * v.rt;
+  l.cols = v.kind == 9 ? 4u * v.nt : (v.kind == 7 && v.pf == 2 ? 8u : 16u) * v.nt;
+  l.threads = v.w * 64u;
+  uint32_t k_groups = 0; // of the wide-K-step body's 8 waves
+  if (matmul_wide(v, nsb)) {
+    k_groups = v.kind == 5 ? 4u : 8u / v.w;
+  } else if (v.kind == 7 && v.nt == 2) {
+    // Past one 16-row block per CU, while one round of 32 x 32 tiles covers
+    // the grid (4096 x 4096 x 64 9.1 us against 12.4, 4096 x 1024 x 64 6.1
+    // against 10.4, 1024 x 4096 x 250 8.8 against 12.0, A/B in one run); not
+    // before (4096 x 4096 x 32 8.6 against 7.3).
+    if (groups(16, 32) > kMatmulCus && groups(32, 32) <= kMatmulCus) k_groups = 8;
+  } else if (v.kind == 5 && v.rt == 4 && v.nt == 1) {
+    // 32 x 32 tiles dequantise half of what 64 x 16 do (4096 x 14336 x 64 22
+    // us against 39), but half their columns are empty up to 16.
+    if (batch > 16) k_groups = 8;
+    l.threads = 512; // the kernel's; four of the waves end at once
+  }
+  if (k_groups == 8) {
+    l.rows = l.cols = 32;
+    l.second = 1;
+  }
+  if (k_groups) {
+    l.threads = 512;
+    // per step and K group 128 bytes of each column: 16 KiB (6 buffers, with
+    // 144 bytes of each wave's 32 rows), 32 KiB (4) or 64 KiB (2, with 128)
+    l.lds = k_groups * l.cols == 128u ? 6u * 16384u + 8u * 32u * 144u
+                                      : 4u * 32768u + 8u * 32u * 128u;
+  } else {
+    // kind 5 sums the partial tiles of its waves in LDS (one 16x16 f32 tile =
+    // 1 KiB per wave); kind 7: 128 KiB of X staging (64 KiB with 8-column
+    // groups), whose wave regions then hold the waves' partial tiles
+    l.lds = v.kind == 5   ? kx_lds_bytes(v)
+            : v.kind == 7 ? (v.pf == 2 ? 65536u : 131072u)
+            : v.kind == 8 ? rm_lds_bytes(v)
+            : v.kind == 9 ? lk_lds_bytes(v)
+                          : 0u;
+  }
+  return l;
+}
+
 static MatmulVariant q4k_matmul_default(uint32_t n_rows, uint32_t batch, uint32_t nsb) {
   const auto groups = [&](uint32_t rows_per_wg, uint32_t cols_per_wg) {
     return (uint64_t)((n_rows + rows_per_wg - 1) / rows_per_wg) *
@@ -1663,9 +1732,9 @@ static MatmulVariant q4k_matmul_default(uint32_t n_rows, uint32_t batch, uint32_
     if (per_group * ((batch + 7u) / 8u) <= kMatmulCus) return {7, 8, 1, 2, 0};
     if (per_group * ((batch + 15u) / 16u) <= kMatmulCus) return {7, 8, 1, 1, 0};
     if (per_group * ((batch + 31u) / 32u) <= kMatmulCus) return {7, 8, 2, 1, 0};
-    // Up to two blocks of 32 columns per CU it still beats the tiles (4096 x
-    // 4096 x 64 13.8 us against 14.7; 2048 x 4096 x 128 13.5 against 14.9),
-    // not at four (8192 x 4096 x 64 18.6 against 16.3).
+    // Up to two blocks of 32 columns per CU it still beats the tiles, as one
+    // 32-row block (4096 x 4096 x 64 10.4 us against 12.8; 2048 x 4096 x 128
+    // 9.5 against 12.2), not at four (8192 x 4096 x 64 16.5 against 14.5).
     if (groups(16, 32) <= 2 * kMatmulCus) return {7, 8, 2, 1, 0};
   }
   // Long rows (K > 4096) over few of them, up to 32 columns: kind 9 (8 waves
@@ -1779,9 +1848,11 @@ static axh_status plan_q4k_matmul(uint32_t n_rows, uint32_t sb_per_row, uint32_t
         std::snprintf(name, cap, "axh_q4k_matmul_ks_k%u_n%u_p%u%s", v.w, v.nt, v.pf,
                       v.rt == 1 ? "_r1" : "");
       else if (v.kind == 5)
-        std::snprintf(name, cap, "axh_q4k_matmul_kx_r%u_n%u_k%u_p%u", v.rt, v.nt, v.w, v.pf);
+        std::snprintf(name, cap, "axh_q4k_matmul_kx_r%u_n%u_k%u_p%u%s", v.rt, v.nt, v.w, v.pf,
+                      matmul_short(v, sb_per_row) ? "_short" : "");
       else if (v.kind == 8)
-        std::snprintf(name, cap, "axh_q4k_matmul_rm_w%u_r%u_p4", v.w, v.rt);
+        std::snprintf(name, cap, "axh_q4k_matmul_rm_w%u_r%u_p4%s", v.w, v.rt,
+                      matmul_short(v, sb_per_row) ? "_short" : "");
       else if (v.kind == 9) {
         if (sb_per_row >= kLkMaxSb)
           return fail(AXH_ERR_INVALID_ARGUMENT,
@@ -1842,36 +1913,23 @@ axh_status axh_q4k_matmul_f16(axh_context *ctx, const void *q, const uint16_t *x
   char name[64];
   s = plan_q4k_matmul(n_rows, sb_per_row, batch, variant, &v, name, sizeof(name));
   if (s != AXH_OK) return s;
-  // kind 5 sums the partial tiles of its waves in LDS (one 16x16 f32 tile =
-  // 1 KiB per wave); kind 7: 128 KiB of X staging (64 KiB with 8-column
-  // groups), whose wave regions then hold the waves' partial tiles
-  const uint32_t lds = v.kind == 5   ? kx_lds_bytes(v)
-                       : v.kind == 7 ? (v.pf == 2 ? 65536u : 131072u)
-                       : v.kind == 8 ? rm_lds_bytes(v)
-                       : v.kind == 9 ? lk_lds_bytes(v)
-                                     : 0u;
-  if (lds > ctx->core->max_lds)
+  const MatmulLaunch l = matmul_launch_of(v, n_rows, batch, sb_per_row);
+  if (l.lds > ctx->core->max_lds)
     return fail(AXH_ERR_INVALID_ARGUMENT, "matmul variant needs more LDS than the device has");
-  const uint32_t tm = v.kind == 3   ? 16u * v.rt
-                      : v.kind == 5 ? 16u * v.rt
-                      : v.kind == 7 ? 16u
-                      : v.kind == 9 ? 16u * v.rt
-                                    : 32u * v.rt * v.w;
-  const uint32_t tn = v.kind == 9 ? 4u * v.nt : (v.kind == 7 && v.pf == 2 ? 8u : 16u) * v.nt;
-  uint64_t gx = (n_rows + tm - 1) / tm;
-  const uint64_t gy = (batch + tn - 1) / tn;
+  uint64_t gx = (n_rows + l.rows - 1) / l.rows;
+  const uint64_t gy = (batch + l.cols - 1) / l.cols;
   if (gx > ctx->core->max_wg[0] || gy > ctx->core->max_wg[1])
     return fail(AXH_ERR_WORKGROUP_COUNT_EXCEEDS_LIMIT, "matmul grid exceeds the device limit");
   hipSetDevice(ctx->core->device);
   axh_kernel *k = nullptr;
-  s = builtin_kernel(ctx, name, 3, sizeof(MatmulArgs), v.w * 64u, &k);
+  s = builtin_kernel(ctx, name, 3, sizeof(MatmulArgs), l.threads, &k);
   if (s != AXH_OK) return s;
   // kind 7 is persistent: one workgroup per CU per column group, even where two would fit
-  if (v.kind == 7 && ctx->core->cu_count < gx) gx = ctx->core->cu_count;
+  if (v.kind == 7 && !l.second && ctx->core->cu_count < gx) gx = ctx->core->cu_count;
   const uint32_t grid[3] = {(uint32_t)gx, (uint32_t)gy, 1};
   void *bufs[3] = {const_cast<void *>(q), const_cast<uint16_t *>(x), y};
-  MatmulArgs a{n_rows, sb_per_row, batch, 0};
-  s = launch_raw(k, grid, bufs, 3, &a, sizeof(a), (uint32_t)lds, pick_stream(ctx, stream));
+  MatmulArgs a{n_rows, sb_per_row, batch, l.second};
+  s = launch_raw(k, grid, bufs, 3, &a, sizeof(a), l.lds, pick_stream(ctx, stream));
   return s == AXH_OK ? ok() : s;
 }
 

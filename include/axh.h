@@ -460,12 +460,17 @@ typedef struct axh_q4_matmul_variant {
                                      chunks through LDS); 0 = default, chosen by the grid
                                      each kind launches on 256 CUs.  Kinds 1, 2, 4
                                      and 6 were removed (no shape where they won) */
-    uint32_t waves_per_workgroup; /* 3, 5, 7, 9: waves splitting K; 8: waves of row_tiles
-                                     row tiles each */
+    uint32_t waves_per_workgroup; /* 3, 7, 9: waves splitting K; 5: parts of K; 8: row
+                                     parts of row_tiles row tiles each.  The main
+                                     forms of kinds 5 and 8 run 8 waves whatever this
+                                     says: rows or parts of K for each wave */
     uint32_t col_tiles;           /* 16-column MFMA tiles per workgroup (kind 8: 8;
-                                     kind 9: 4-column groups, 1, 2 or 4) */
+                                     kind 9: 4-column groups, 1, 2 or 4; kind 5 with
+                                     1: 64 rows x 16 columns up to 16 columns, 32 x
+                                     32 beyond) */
     uint32_t prefetch;            /* K steps in flight (kinds 3, 7; kind 7 prefetch 2:
-                                     8-column groups), LDS ring depth (5, 8: 4), X
+                                     8-column groups), LDS ring depth (5, 8: 4; the
+                                     main forms have their own), X
                                      chunks in flight (9) */
     uint32_t row_tiles;           /* kind 3: 16-row MFMA tiles (0: 2); kind 5: 16-row
                                      MFMA tiles per wave (0: 4); kind 8: 32-row tiles
