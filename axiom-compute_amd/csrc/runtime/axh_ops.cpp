@@ -1783,24 +1783,48 @@ static MatmulVariant q4k_matmul_default(uint32_t n_rows, uint32_t batch, uint32_
   const bool lk_ok = nsb > kSrMaxSb && nsb < kLkMaxSb;
   if (groups(16, 16) <= kMatmulCus) return lk_ok ? MatmulVariant{9, 8, 4, 1, 1} : MatmulVariant{3, 8, 1, 1, 1};
   if (groups(32, 16) <= kMatmulCus) return lk_ok ? MatmulVariant{9, 8, 4, 1, 2} : MatmulVariant{3, 8, 1, 1, 2};
-  // kind 8 (32 x 32 MFMA tiles) where its rows fill the chip: 14336 x 4096 x
-  // 512 74.1 us (8 waves of 32 rows) against 83-94 for a row-split kind,
-  // B = 256 49.3 (4 waves of 32 rows) against 52.1; 8192 x 4096 x 512 46.0 us
-  // with 4 waves against 60.7 as K-split tiles.
-  if (batch > 256 && groups(256, 128) >= kMatmulFill) return {8, 8, 8, 4, 1};
-  // from 128 columns (A/B in one run against the K-split tile kind at 128
-  // columns: 20480 x 4096 40.35 vs 51.0 us, 28672 x 4096 43.95 vs 53.0, 28672
-  // x 8192 78.45 vs 94.92, 24576 x 14336 136.0 vs 156.2; below the fill
-  // 16384 x 8192 and 11008 x 4096 stay on the K-split tile kind)
-  if (batch >= 128 && groups(128, 128) >= kMatmulFill) return {8, 4, 8, 4, 1};
-  // The K-split tile kind: up to 128 columns per workgroup, halved until the
-  // grid fills (4096 x 14336 x 64: one column tile 41.3 us against four
-  // 58.8; 4096 x 11008 x 128: two 37.9 against eight 76.5).  Two column
-  // tiles prefetch 3 steps at K > 4096 (4096 x 14336 x 128 45.8 us against
-  // 47.6), 2 at K <= 4096 (4096 x 4096 x 128 16.0 against 16.3).
-  uint32_t nt = batch <= 16 ? 1u : batch <= 32 ? 2u : batch <= 64 ? 4u : 8u;
-  while (nt > 1 && groups(64, 16 * nt) < kMatmulFill) nt /= 2;
-  return {5, 4, nt, nt == 1 || (nt == 2 && nsb > kSrMaxSb) ? 3u : 2u, 4};
+  // kind 8 (128 columns per workgroup) from 128 columns where its rows fill
+  // the chip: 128-row tiles while one round of them covers the grid (14336 x
+  // 4096 x 256 36.5 us, against 42 before they split K), then 256-row tiles
+  // (28672 x 4096 x 256 67.6 us against 83.6 with 128-row tiles in two rounds,
+  // 40960 x 4096 x 128 60.5 against 69, 18432 x 4096 x 256 62.2 against 66.3).
+  // Below the fill the K-split tiles are ahead (11008 x 4096 x 128).
+  if (batch >= 128 && groups(128, 128) >= kMatmulFill)
+    return groups(128, 128) > kMatmulCus ? MatmulVariant{8, 8, 8, 4, 1}
+                                         : MatmulVariant{8, 4, 8, 4, 1};
+  // Kind 5 beyond: the narrowest of its tiles whose grid is one round, since a
+  // second round doubles the time whatever it holds.  32 x 32 (the second body
+  // of the one-column-tile kernel): 4096 x 14336 x 64 22 us against 39 as 64 x
+  // 16 and 47 in 64 x 32 tiles, 8192 x 14336 x 32 25.7 against 42.  64 x 32
+  // while they fit: 5000 x 11008 x 77 30 us against 35 in 64 x 64 tiles.  64 x
+  // 64: 5000 x 11008 x 128 34.5 against 50.9 in two rounds of 64 x 32.  Then 64
+  // x 128 (8192 x 8192 x 256 46 us in one round, against 52 as four-wave
+  // tiles), or the widest tile the columns fill.
+  if (batch > 16 && groups(32, 32) <= kMatmulCus) return {5, 4, 1, 3, 4};
+  if (batch <= 8) return {5, 4, 1, 3, 4}; // 64 x 16 (14336 x 14336 x 8 40 us)
+  // 11008 x 11008 x 9 to 16 28 us in 64 x 32 tiles, 30 to 31.5 in 64 x 16
+  uint32_t nt = 2;
+  while (nt < 8 && 16 * nt < batch && groups(64, 16 * nt) > kMatmulCus) nt *= 2;
+  return {5, 4, nt, nt == 2 && nsb > kSrMaxSb ? 3u : 2u, 4};
+}
+
+// The holes a caller's variant leaves 0 while it names others: the default's,
+// with kind 8's waves and kind 5's column tiles by a rule of their own, so that
+// a partial variant means (and is accepted or refused) the same wherever the
+// line between the default's tiles lies.
+static MatmulVariant q4k_matmul_holes(uint32_t n_rows, uint32_t batch, uint32_t nsb) {
+  const auto groups = [&](uint32_t rows_per_wg, uint32_t cols_per_wg) {
+    return (uint64_t)((n_rows + rows_per_wg - 1) / rows_per_wg) *
+           ((batch + cols_per_wg - 1) / cols_per_wg);
+  };
+  MatmulVariant v = q4k_matmul_default(n_rows, batch, nsb);
+  if (v.kind == 8) v.w = batch > 256 && groups(256, 128) >= kMatmulFill ? 8u : 4u;
+  if (v.kind == 5) {
+    v.nt = batch <= 16 ? 1u : batch <= 32 ? 2u : batch <= 64 ? 4u : 8u;
+    while (v.nt > 1 && groups(64, 16 * v.nt) < kMatmulFill) v.nt /= 2;
+    v.pf = v.nt == 1 || (v.nt == 2 && nsb > kSrMaxSb) ? 3u : 2u;
+  }
+  return v;
 }
 
 uint32_t axh_q4k_matmul_variant_count(void) {
@@ -1822,7 +1846,9 @@ static axh_status plan_q4k_matmul(uint32_t n_rows, uint32_t sb_per_row, uint32_t
                                   const axh_q4_matmul_variant *variant, MatmulVariant *out,
                                   char *name, size_t cap) {
   MatmulVariant want = q4k_matmul_default(n_rows, batch, sb_per_row);
-  if (variant) {
+  if (variant && (variant->kind || variant->waves_per_workgroup || variant->col_tiles ||
+                  variant->prefetch || variant->row_tiles)) {
+    want = q4k_matmul_holes(n_rows, batch, sb_per_row);
     if (variant->kind && variant->kind != want.kind) {
       want.kind = variant->kind;
       want.rt = 0; // the row tiles of the requested kind's default

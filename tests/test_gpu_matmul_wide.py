@@ -48,6 +48,28 @@ def test_tiles_and_k_groups_at_their_edges(ctx, axc, rows, sb, batch):
         _check(ctx, axc, rows, sb, batch, axc.MatmulVariant(*v))
 
 
+# either side of the lines between the default's tiles (256 and 257 workgroups)
+@pytest.mark.parametrize("rows,sb,batch,kernel", [
+    (8192, 17, 17, "kx_r4_n1_k4_p3"),          # 32 x 32 tiles: 256
+    (8193, 17, 17, "kx_r4_n2_k4_p3"),          # 257
+    (8193, 17, 16, "kx_r4_n2_k4_p3"),          # past the long-rows kind, 16 columns
+    (4096, 5, 33, "sr_w8_s2_n2"),              # two 16-row blocks per CU: 256 of 32 rows
+    (2049, 16, 97, "kx_r4_n2_k4_p2"),          # 65 x 4 of 32 rows is one more
+    (8192, 7, 33, "kx_r4_n2_k4_p2_short"),     # 128 x 2 of 64 x 32
+    (8193, 7, 33, "kx_r4_n4_k4_p2_short"),
+    (4097, 17, 128, "kx_r4_n4_k4_p2"),         # 65 x 4 of 64 x 32
+    (16385, 8, 64, "kx_r4_n4_k4_p2"),          # none fits one round: the widest filled
+    (16385, 7, 65, "kx_r4_n8_k4_p2_short"),
+    (16385, 8, 65, "kx_r4_n8_k4_p2"),
+    (32768, 3, 128, "rm_w4_r1_p4_short"),
+    (32768, 4, 128, "rm_w4_r1_p4"),
+    (32769, 1, 128, "rm_w8_r1_p4"),
+])
+def test_default_tiles(ctx, axc, rows, sb, batch, kernel):
+    assert axc.q4k_matmul_kernel_name(rows, sb, batch) == "axh_q4k_matmul_" + kernel
+    _check(ctx, axc, rows, sb, batch)
+
+
 # either side of the line between the short and the wide K steps
 @pytest.mark.parametrize("rows,sb,variant,kernel", [
     (300, 7, (5, 4, 8, 2, 4), "kx_r4_n8_k4_p2_short"), (300, 8, (5, 4, 8, 2, 4), "kx_r4_n8_k4_p2"),
@@ -65,3 +87,12 @@ def test_streaming_rows_second_body_line(ctx, axc):
     goes to 32-row tiles while those are one round, in every K remainder."""
     for rows, sb, batch in [(4096, 16, 32), (4097, 16, 32), (2064, 7, 64), (1024, 1, 250)]:
         _check(ctx, axc, rows, sb, batch, axc.MatmulVariant(7, 8, 2, 1))
+
+
+def test_partial_variants_keep_their_holes(axc):
+    """Holes a caller leaves 0 beside others do not follow the default's lines."""
+    name = axc.q4k_matmul_kernel_name
+    assert name(28672, 16, 256) == "axh_q4k_matmul_rm_w8_r1_p4"
+    assert name(28672, 16, 256, axc.MatmulVariant(row_tiles=2)) == "axh_q4k_matmul_rm_w4_r2_p4"
+    assert name(5000, 43, 128) == "axh_q4k_matmul_kx_r4_n4_k4_p2"
+    assert name(5000, 43, 128, axc.MatmulVariant(col_tiles=1)) == "axh_q4k_matmul_kx_r4_n1_k4_p3"
