@@ -853,6 +853,13 @@ __device__ __forceinline__ void q4k_matvec_flat(const uint8_t *__restrict__ q,
 // instances for rows of up to 16 superblocks are (axh_q5k_matvec_one_i{NIT},
 // see the runtime's Q5_K kernel choice).
 //
+// nw (8 to 12; 0: 8): the waves of the launch, 2 * nw rows per workgroup.  The
+// waves past the eighth stage the start of the next chunk, the values that it is
+// staged with an iteration later, before any wave reads it (a guard around
+// their loads and stores measured slower: Q4_K 8192 x 5376 with 8 waves 7.97 us
+// against 7.24).  Just past 16 rows per CU a second workgroup on some of
+// the CUs doubles their time, one larger workgroup per CU spreads the rows.
+//
 // kWhole (axh_q4k_matvec_onex_i{NIT}): x is staged whole first, behind one
 // barrier, with the first iteration's weights already requested, and the
 // early-refill loop then runs without barriers, so the waves of a workgroup
@@ -895,7 +902,8 @@ template <int NIT, bool kDual = false, bool kQ5 = false, bool kWhole = false, in
 __device__ __forceinline__ void q4k_matvec_one(const uint8_t *__restrict__ q,
                                                const uint8_t *__restrict__ q2,
                                                const float *__restrict__ x, float *__restrict__ y,
-                                               uint32_t n_rows, uint32_t nsb, float *lds) {
+                                               uint32_t n_rows, uint32_t nsb, float *lds,
+                                               uint32_t nw = 8u) {
   constexpr int NW = 8, NT = NW * 64;
   constexpr int RPW = kDual ? 2 : 1; // row slots per lane: (gate, up) or one row
   const uint32_t tid = threadIdx.x;
@@ -906,7 +914,7 @@ __device__ __forceinline__ void q4k_matvec_one(const uint8_t *__restrict__ q,
   // the first and of the second matrix, one row per lane slot, so the pair's
   // loads go through one wave-uniform resource each; W is the pair index.
   static_assert(!(kPair && kDual), "one pairing of gate and up rows");
-  const uint32_t W = kPair ? (blockIdx.x * NW + wave) >> 1 : blockIdx.x * NW + wave;
+  const uint32_t W = kPair ? (blockIdx.x * NW + wave) >> 1 : blockIdx.x * (nw ? nw : 8u) + wave;
   const bool mine = W < (n_rows + 1u) >> 1; // this wave has a pair of rows
   static_assert(!(kQ40 && (kDual || kQ5)), "Q4_0 rows are a layout of their own");
   // kQ40: nsb is the row's Q4_0 block count, read as octets of 8 blocks.
@@ -988,17 +996,17 @@ __device__ __forceinline__ void q4k_matvec_one(const uint8_t *__restrict__ q,
 }
 
 #define AXH_Q4K_MATVEC_ONE(NIT)                                                                  \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q4k_matvec_one_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,      \
                                 float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
-    q4k_matvec_one<NIT>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn);                     \
+    q4k_matvec_one<NIT>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn, a.pad);              \
   }                                                                                              \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q4k_matvec_onex_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
-    q4k_matvec_one<NIT, false, false, true>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn); \
+    q4k_matvec_one<NIT, false, false, true>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn, a.pad);\
   }
 AXH_Q4K_MATVEC_ONE(1)
 AXH_Q4K_MATVEC_ONE(2)
@@ -1018,19 +1026,19 @@ AXH_Q4K_MATVEC_ONE(15)
 AXH_Q4K_MATVEC_ONE(16)
 
 #define AXH_Q5K_MATVEC_ONE(NIT)                                                                  \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q5k_matvec_one_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,      \
                                 float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
-    q4k_matvec_one<NIT, false, true>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn);        \
+    q4k_matvec_one<NIT, false, true>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn, a.pad); \
   }
 #define AXH_Q5K_MATVEC_ONEP(NIT)                                                                 \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q5k_matvec_onep_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;        \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT, false, true, false, 2>(q, q, x, y, a.n_rows, a.units_per_row,            \
-                                               axh_lds_dyn);                                     \
+                                               axh_lds_dyn, a.pad);                              \
   }
 AXH_Q5K_MATVEC_ONE(1)
 AXH_Q5K_MATVEC_ONE(2)
@@ -1048,12 +1056,12 @@ AXH_Q5K_MATVEC_ONE(8)
 AXH_Q5K_MATVEC_ONEP(8)
 
 #define AXH_Q4K_MATVEC_ONEP(NIT)                                                                 \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q4k_matvec_onep_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT, false, false, false, 2>(q, q, x, y, a.n_rows, a.units_per_row,           \
-                                                axh_lds_dyn);                                    \
+                                                axh_lds_dyn, a.pad);                             \
   }
 AXH_Q4K_MATVEC_ONEP(3)
 AXH_Q4K_MATVEC_ONEP(4)
@@ -1451,8 +1459,8 @@ __device__ __forceinline__ void q6k_stage_chunk(float *xs, float *ss, uint32_t t
 }
 
 // Q6_K one pass, one pair of rows per wave (axh_q6k_matvec_one_i{NIT}): rows
-// of 8 * (NIT - 1) < nsb <= 8 * NIT superblocks, 8 waves per workgroup, wave
-// W takes rows 2W and 2W + 1, one workgroup per 16 rows, all launched.  The
+// of 8 * (NIT - 1) < nsb <= 8 * NIT superblocks, 8 to 12 waves per workgroup
+// (nw), wave W takes rows 2W and 2W + 1, all workgroups launched.  The
 // Q4_K one-pass order (q4k_matvec_one) with the Q6_K loads and decode of the
 // persistent kernel, so its output equals the persistent kernel's bit for
 // bit: x staged chunk by chunk (8 superblocks, 8 KiB) with the next
@@ -1464,14 +1472,15 @@ __device__ __forceinline__ void q6k_stage_chunk(float *xs, float *ss, uint32_t t
 template <int NIT, int XD>
 __device__ __forceinline__ void q6k_matvec_one(const uint8_t *__restrict__ q,
                                                const float *__restrict__ x, float *__restrict__ y,
-                                               uint32_t n_rows, uint32_t nsb, float *lds) {
+                                               uint32_t n_rows, uint32_t nsb, float *lds,
+                                               uint32_t nw) {
   constexpr int NW = 8, NT = NW * 64;
   static_assert(XD == 1 || XD == 2, "x one or two chunks ahead");
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t G = lane >> 2, half = G >> 3, s = G & 7u, c = lane & 3u;
-  const uint32_t W = blockIdx.x * NW + wave;
+  const uint32_t W = blockIdx.x * (nw ? nw : 8u) + wave;
   const bool mine = W < (n_rows + 1u) >> 1; // this wave has a pair of rows
   // The host guarantees n_rows * row_bytes < 2^32 for this kernel.
   const uint32_t row_bytes = nsb * kQ6kSbBytes;
@@ -1503,12 +1512,12 @@ __device__ __forceinline__ void q6k_matvec_one(const uint8_t *__restrict__ q,
 }
 
 #define AXH_Q6K_MATVEC_ONE(NIT, XD, TAG)                                                         \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q6k_matvec_one##TAG##_i##NIT(const uint8_t *__restrict__ q,                            \
                                        const float *__restrict__ x, float *__restrict__ y,       \
                                        AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;                         \
     extern __shared__ float axh_lds_dyn[];                                                       \
-    q6k_matvec_one<NIT, XD>(q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn);                    \
+    q6k_matvec_one<NIT, XD>(q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn, a.pad);             \
   }
 AXH_Q6K_MATVEC_ONE(1, 1, )
 AXH_Q6K_MATVEC_ONE(2, 1, )
@@ -2409,27 +2418,27 @@ AXH_Q4_0_MATVEC_FLAT(1, 16, 2, 1)
 // 64 * (NIT - 1) < nb <= 64 * NIT blocks (x chunk by chunk, x whole, x two
 // chunks ahead).
 #define AXH_Q4_0_MATVEC_ONE(NIT)                                                                 \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q4_0_matvec_one_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;        \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT, false, false, false, 1, true>(q, q, x, y, a.n_rows, a.units_per_row,     \
-                                                      axh_lds_dyn);                              \
+                                                      axh_lds_dyn, a.pad);                       \
   }                                                                                              \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q4_0_matvec_onex_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,    \
                                   float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;       \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT, false, false, true, 1, true>(q, q, x, y, a.n_rows, a.units_per_row,      \
-                                                     axh_lds_dyn);                               \
+                                                     axh_lds_dyn, a.pad);                        \
   }
 #define AXH_Q4_0_MATVEC_ONEP(NIT)                                                                \
-  extern "C" __global__ void __launch_bounds__(512)                                              \
+  extern "C" __global__ void __launch_bounds__(768)                                              \
       axh_q4_0_matvec_onep_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,    \
                                   float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;       \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT, false, false, false, 2, true>(q, q, x, y, a.n_rows, a.units_per_row,     \
-                                                      axh_lds_dyn);                              \
+                                                      axh_lds_dyn, a.pad);                       \
   }
 AXH_Q4_0_MATVEC_ONE(1)
 AXH_Q4_0_MATVEC_ONE(2)

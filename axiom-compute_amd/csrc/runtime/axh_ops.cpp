@@ -137,7 +137,10 @@ bool is_builtin_code_object(const void *co, size_t bytes) {
 axh_status builtin_kernel(axh_context *ctx, const char *entry, uint32_t n_buffers,
                           uint32_t pc_bytes, uint32_t wg_x, axh_kernel **out) {
   std::lock_guard<std::mutex> lk(ctx->ops_mu);
-  auto it = ctx->ops.find(entry);
+  // a kernel of more than 512 threads may be launched with several sizes
+  std::string key(entry);
+  if (wg_x > 512u) key += "@" + std::to_string(wg_x);
+  auto it = ctx->ops.find(key);
   if (it != ctx->ops.end()) {
     *out = it->second;
     return AXH_OK;
@@ -164,7 +167,7 @@ axh_status builtin_kernel(axh_context *ctx, const char *entry, uint32_t n_buffer
   axh_kernel *k = nullptr;
   axh_status s = axh_prepare_kernel(ctx, co, n, &plan, pc_bytes, entry, &k);
   if (s != AXH_OK) return s;
-  ctx->ops.emplace(entry, k);
+  ctx->ops.emplace(std::move(key), k);
   *out = k;
   return AXH_OK;
 }
@@ -503,6 +506,22 @@ static bool q4k_tiled_few(uint32_t n_rows, uint32_t nsb) {
   return nsb >= (n_rows <= kTiledFewShortMaxRows ? kTiledFewShortMinSb : kTiledFewMidMinSb);
 }
 
+// Waves of a one-pass workgroup (two rows each).  Past 4096 rows 8 waves would
+// need a second workgroup on some CUs, which then take twice as long as the
+// rest (Q4_K 4096 x 14336 8.2 us, 4352 x 14336 12.2); up to 12 waves, one
+// workgroup per CU takes them all.  us before -> with 9 to 12 waves, A/B in one
+// run: 4352, 4999 and 6144 rows, Q4_K x 14336 12.2 -> 10.1, 12.3 -> 10.3, 13.3
+// -> 11.4, x 5376 6.35 -> 5.62, 6.42 -> 5.76, 6.61 -> 6.17, x 4096 4.75 ->
+// 4.49, 4.88 -> 4.60, 4.98 -> 4.90; Q5_K x 4096 6.32 -> 5.78, 6.42 -> 5.97,
+// 6.54 -> 6.33; Q6_K x 5376 9.25 -> 8.00, 9.36 -> 8.34, 9.61 -> 9.14; Q4_0 x
+// 14336 11.9 -> 9.42, 12.2 -> 10.8, 13.8 -> 11.0.  With 14 and 16 waves two
+// workgroups of 8, whose barriers do not stop each other, are ahead (Q4_K 7168
+// x 5376 6.83 against 7.22, 8192 x 5376 7.11 against 8.32).
+static uint32_t one_pass_waves(uint32_t n_rows) {
+  const uint32_t pairs = n_rows / 2u + n_rows % 2u, w = (pairs + 255u) / 256u;
+  return w > 8u && w <= 12u ? w : 8u;
+}
+
 static bool use_one_pass(uint32_t n_rows, uint32_t nsb) {
   if (nsb < 1 || nsb > kOneMaxSb || n_rows < kOneMinRows) return false;
   return n_rows <= kOneMaxRows || (nsb <= kOneTallMaxSb && n_rows <= kOneTallMaxRows);
@@ -631,11 +650,11 @@ static axh_status plan_q4k(uint32_t n_rows, uint32_t sb_per_row, const axh_q4_va
                            (xd == 2u || (xd == 0u && nit >= kOnePMinIt && n_rows <= kOnePMaxRows));
     std::snprintf(p->name, sizeof(p->name), "axh_q4k_matvec_one%s_i%u",
                   fam == AXH_Q4K_FAMILY_ONE_PASS_X ? "x" : two_ahead ? "p" : "", nit);
-    p->nw = 8;
+    p->nw = one_pass_waves(n_rows);
     p->lds = nsb * 1120u;
-    p->flat = false; // one workgroup per 16 rows, all of them launched
-    p->units = (n_rows + 15u) / 16u;
-    p->args = RowsArgs{n_rows, nsb, nsb, 0};
+    p->flat = false; // one workgroup per 2 * nw rows, all of them launched
+    p->units = ((n_rows + 1u) / 2u + p->nw - 1u) / p->nw;
+    p->args = RowsArgs{n_rows, nsb, nsb, p->nw};
     return ok();
   }
   case AXH_Q4K_FAMILY_TILED: {
@@ -1109,8 +1128,10 @@ constexpr uint32_t kKqOneMaxIt = 8; // one-pass kernels compiled for 1-8 steps
 // persistent: 256 x 4096 4.05 vs 4.74, 512 x 4096 4.56 vs 4.65, 1024 x 4096
 // 4.62 vs 4.85, 2048 x 4096 4.85 vs 5.00, 4096 x 4096 5.44 vs 5.90, 4096 x
 // 3072 5.21 vs 5.38, 4096 x 2048 3.72 vs 4.30, 1024 x 2048 3.24 vs 4.08; but
-// 6144 x 4096 7.28 vs 6.91 and 14336 x 4096 12.08 vs 11.95.
-constexpr uint32_t kQ6OneMinRows = 256, kQ6OneMaxRows = 4096;
+// 6144 x 4096 7.28 vs 6.91 and 14336 x 4096 12.08 vs 11.95.  With up to 10
+// waves per workgroup (one_pass_waves) it holds to 5120 rows: 4352 x 4096 6.15
+// vs 6.51, 4999 x 4096 6.44 vs 6.57; 6144 x 4096 7.06 vs 6.82.
+constexpr uint32_t kQ6OneMinRows = 256, kQ6OneMaxRows = 4096, kQ6OneWavesMaxRows = 5120;
 
 // Longer rows take the one-pass kernel past 2048 rows too: Q5_K 2049-4096
 // rows of 17-64 superblocks (4096 x 6144 5.67 vs 6.49 us, 4096 x 10240 7.84 vs
@@ -1120,11 +1141,22 @@ constexpr uint32_t kQ6OneMinRows = 256, kQ6OneMaxRows = 4096;
 // 8192 x 10240 15.24 vs 15.71; 4096 x 14336 11.79 vs 11.52 stays persistent).
 // At 2048 rows the 4-wave persistent kernel stays ahead (Q5_K 2048 x 14336
 // 7.64 vs 9.18).
+// Over 4113-6144 rows one workgroup of 9 to 12 waves per CU (one_pass_waves) is
+// ahead for all of 17-64 superblocks: 4352, 4999 and 6144 rows, Q5_K x 5376
+// 7.18, 7.30, 7.83 vs 8.00, 8.08, 8.35, x 14336 13.6, 14.2, 15.2 vs 17.4, 17.3,
+// 17.3; Q6_K x 14336 14.5, 16.4, 17.5 vs 18.6, 18.8, 18.9.  Up to 4112 rows, one
+// 8-wave workgroup past one per CU, the persistent kernel stays: the tests name
+// it at 4097.
 constexpr uint32_t kKqOneLongMinRows = 2049, kQ5OneLongMaxRows = 4096, kQ6OneLongMaxRows = 8192;
 constexpr uint32_t kQ5OneLongMaxSb = 64, kQ6OneLongMaxSb = 40;
+constexpr uint32_t kKqOneWavesMinRows = 4113, kKqOneWavesMaxRows = 6144;
 
 static bool kq_one_long(const KqFormat &f, uint32_t n_rows, uint32_t nsb) {
   const bool q5 = &f == &kQ5kFormat;
+  if (n_rows >= kKqOneWavesMinRows &&
+      (nsb > kKqOneMaxSb ? n_rows <= kKqOneWavesMaxRows && nsb <= kQ5OneLongMaxSb
+                         : n_rows <= kQ6OneWavesMaxRows))
+    return true;
   return n_rows >= kKqOneLongMinRows && nsb > kKqOneMaxSb &&
          n_rows <= (q5 ? kQ5OneLongMaxRows : kQ6OneLongMaxRows) &&
          nsb <= (q5 ? kQ5OneLongMaxSb : kQ6OneLongMaxSb);
@@ -1162,11 +1194,11 @@ static axh_status plan_kq(const KqFormat &f, uint32_t n_rows, uint32_t sb_per_ro
     if (xd == 2u && nit < 3u)
       return fail(AXH_ERR_INVALID_ARGUMENT, "x two chunks ahead needs three or more steps");
     std::snprintf(p->name, sizeof(p->name), "%s%s_i%u", f.one_prefix, xd == 2u ? "p" : "", nit);
-    p->nw = 8;
+    p->nw = one_pass_waves(n_rows);
     p->lds = sb_per_row * f.lds_per_sb;
-    p->flat = false; // one workgroup per 16 rows, all of them launched
-    p->units = (n_rows + 15u) / 16u;
-    p->args = RowsArgs{n_rows, sb_per_row, sb_per_row, 0};
+    p->flat = false; // one workgroup per 2 * nw rows, all of them launched
+    p->units = ((n_rows + 1u) / 2u + p->nw - 1u) / p->nw;
+    p->args = RowsArgs{n_rows, sb_per_row, sb_per_row, p->nw};
     return ok();
   }
   if (variant && variant->nontemporal == 1)
@@ -1446,11 +1478,11 @@ static axh_status plan_q4_0(uint32_t n_rows, uint32_t nb, const axh_q4_variant *
                                          n_rows >= kQ4_0OnePMinRows));
     std::snprintf(p->name, sizeof(p->name), "axh_q4_0_matvec_one%s_i%u",
                   fam == AXH_Q4K_FAMILY_ONE_PASS_X ? "x" : two_ahead ? "p" : "", nit);
-    p->nw = 8;
+    p->nw = one_pass_waves(n_rows);
     p->lds = n_oct * 1120u;
-    p->flat = false; // one workgroup per 16 rows, all of them launched
-    p->units = (n_rows + 15u) / 16u;
-    p->args = RowsArgs{n_rows, nb, nb, 0};
+    p->flat = false; // one workgroup per 2 * nw rows, all of them launched
+    p->units = ((n_rows + 1u) / 2u + p->nw - 1u) / p->nw;
+    p->args = RowsArgs{n_rows, nb, nb, p->nw};
     return ok();
   }
   case AXH_Q4K_FAMILY_TILED: {
