@@ -835,9 +835,9 @@ __device__ __forceinline__ void q4k_matvec_flat(const uint8_t *__restrict__ q,
 }
 
 // One pass, one bundle pair per wave (axh_q4k_matvec_one_i{NIT}): rows of
-// 8 * (NIT - 1) < nsb <= 8 * NIT superblocks, 8 waves per workgroup, wave W
+// 8 * (NIT - 1) < nsb <= 8 * NIT superblocks, nw waves per workgroup, wave W
 // takes rows 2W and 2W + 1 and the grid covers all of them, one workgroup per
-// 16 rows.  The persistent kernel's early-refill order (one iteration in
+// 2 * nw rows.  The persistent kernel's early-refill order (one iteration in
 // flight, x staged chunk by chunk with the weights), fully unrolled over the
 // NIT iterations, so no load, barrier or bookkeeping is spent past the row.
 // Every row group stages x itself (nsb KiB per 16 rows), which costs more

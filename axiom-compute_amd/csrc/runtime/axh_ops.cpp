@@ -44,7 +44,10 @@ struct MatmulArgs {
 //   kind 5 (K-split tile) axh_q4k_matmul_kx_r{RT}_n{NT}_k{W}_p{PF}: a 16*RT x 16*NT tile per
 //                       workgroup, its W waves splitting K by 64-wide superblock chunks,
 //                       register A, operands through per-wave LDS rings, PF superblocks in
-//                       flight.
+//                       flight.  r4 with n2, n4 p2 and n8 p2 (from 8 superblocks) and kind
+//                       8's r1 (from 4 at W = 4) run the wide-K-step body of 8 waves
+//                       (matmul_wide); n1 past 16 columns and kind 7's _n2 between one and
+//                       two blocks per CU its 32 x 32 form (matmul_launch_of).
 //   kind 7 (streaming rows) axh_q4k_matmul_sr_w{W}_s2[_n2|_h]: persistent, one workgroup per
 //                       CU over 16-row blocks, K <= 4096 (pf 2: 8-column groups).
 //   kind 8 (32x32 tiles) axh_q4k_matmul_rm_w{W}_r{RT}_p4: W waves of RT 32-row MFMA tiles
@@ -448,7 +451,8 @@ static bool q4k_use_wg(uint32_t n_rows, uint32_t nsb) {
 }
 
 // One pass with one pair of rows per wave (axh_q4k_matvec_one_i{NIT}, NIT =
-// ceil(nsb / 8)): one 8-wave workgroup per 16 rows, all launched, each
+// ceil(nsb / 8)): one 8-wave workgroup per 16 rows (9 to 12 waves over 4097 to
+// 6144 rows, see one_pass_waves), all launched, each
 // staging x for its own rows.  Faster than the persistent kernels from 32 up
 // to 32768 rows (A/B in one run: 4096 x 14336 8.1-8.4 vs 8.5-8.7 us, 4096 x
 // 4096 4.06 vs 4.6-4.9, 14336 x 4096 8.9-9.1 vs 9.9-10.5, 32768 x 4096 17.0
@@ -1667,17 +1671,15 @@ constexpr uint32_t kSrMaxSb = 16;
 
 // The default matmul kind follows the grid each kind would launch, counted in
 // MI355X's 256 CUs (a constant, so that the choice and its kernel name do not
-// depend on the device a query runs on).  Measured over 60 shapes (1024 to
-// 14336 rows, K = 4096 and 14336, 8 to 512 columns, every compiled variant):
-// the choice below is the fastest variant at 59 and within 2% at the last.
-// A later sweep of 22 shapes (up to 28672 rows, K up to 14336) moved two
-// regions: 128 columns on enough rows (32 x 32 tiles) and more than 32
-// columns on few long rows (the long-rows kind).
+// depend on the device a query runs on).  Which kind takes which shape was
+// measured over 82 shapes (1024 to 28672 rows, K = 4096 to 14336, 8 to 512
+// columns, every variant compiled then); the tiles within kinds 5 and 8 again
+// with the wide-K-step bodies (figures at the rules).
 constexpr uint64_t kMatmulCus = 256;
-// Workgroups the tile kinds (5 and 8) need before their tile size matters
-// less than filling the chip: 5/8 of the CUs.  Below it, more and smaller
-// tiles win (4096 x 4096 x 256: 16-row x 64-column K-split tiles in 256
-// workgroups 21.5 us, 32 x 32 MFMA tiles in 64 workgroups 37.6).
+// Workgroups of 128 rows x 128 columns that kind 8 needs, and kind 9 of its own
+// tiles, before a smaller tile fills the chip better: 5/8 of the CUs (4096 x
+// 4096 x 256: 64-row x 64-column tiles in 256 workgroups 21.5 us, kind 8 in 64
+// workgroups 37.6).
 constexpr uint64_t kMatmulFill = 160;
 
 // Whether a kind 5 or 8 variant runs the wide-K-step body: its 8 waves split K
