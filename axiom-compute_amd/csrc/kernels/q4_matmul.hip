@@ -1723,10 +1723,10 @@ extern "C" __global__ void __launch_bounds__(512)
                                float *__restrict__ y, AXH_MATMUL_ARGS) {
   AXH_MATMUL_UNPACK;
   extern __shared__ f32x4_t axh_sr_dyn[];
-  if (a.pad != 0u)
-    q4k_matmul_wk<8, 1>(q, x, y, a, axh_sr_dyn);
-  else
+  if (__builtin_expect(a.pad == 0u, 1))
     q4k_matmul_sr<8, 2, 2, false>(q, x, y, a, axh_sr_dyn);
+  else
+    q4k_matmul_wk<8, 1>(q, x, y, a, axh_sr_dyn);
 }
 
 extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
