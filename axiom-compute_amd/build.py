@@ -43,7 +43,7 @@ HIP_FLAGS = [
 # kernarg load before its first memory request.
 KERNEL_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
-KERNELS = ["q4_matvec", "q4_matmul"]
+KERNELS = ["q4_matvec", "q4_matvec_wide", "q4_matmul"]
 
 # Host-only sanitizer build (g++ lines only).
 SAN_FLAGS = ["-fsanitize=address,undefined", "-fno-omit-frame-pointer",
@@ -81,6 +81,7 @@ def build_runtime(cos: dict[str, Path], sanitize: bool = False) -> Path:
     _run([HIPCC, *HIP_FLAGS, "-fPIC", "-c", "-I", str(ROOT / "include"), "-I", str(rt),
           "-o", str(noalloc_o), str(rt / "axh_noalloc.hip")])
     _run(["gcc", "-c", f'-DAXH_Q4_MATVEC_CO="{cos["q4_matvec"]}"',
+          f'-DAXH_Q4_MATVEC_WIDE_CO="{cos["q4_matvec_wide"]}"',
           f'-DAXH_Q4_MATMUL_CO="{cos["q4_matmul"]}"', "-o", str(embed_o),
           str(rt / "axh_embed.S")])
     out = SAN_LIB if sanitize else LIB

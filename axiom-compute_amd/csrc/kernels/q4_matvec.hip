@@ -1,6 +1,8 @@
 // gfx950 Q4_K_M and Q4_0 dequant-matvec kernels, plus the decode-only kernels
-// used by the bit-exact checks.  Built into one code object (q4_matvec.hsaco)
-// that the runtime loads with hipModuleLoadData.
+// used by the bit-exact checks.  Built into one code object (q4_matvec.co)
+// that the runtime loads with hipModuleLoadData, and, with AXH_WIDE_ONE_PASS
+// defined (q4_matvec_wide.hip), into a second one that holds the one-pass
+// kernels alone, for workgroups of 9 to 12 waves (see kOnePassWide).
 //
 // Kernel argument convention (matches the runtime's binding plans): one
 // pointer per buffer binding in binding order, then one push-constant struct
@@ -14,11 +16,27 @@
 
 using namespace axh;
 
+// One-pass matvecs (q4k_matvec_one, q6k_matvec_one): 8 waves per workgroup, or
+// 9 to 12 of them (RowsArgs.pad) in the wide code object.  For 8 waves the count
+// is a constant, because the workgroup's first row is on the path to the first
+// weight address: with a run-time count in the same kernel, and its larger
+// launch bound, Q4_K 4096 x 14336 took 7.32 us against 7.22, 4096 x 4096 3.27
+// against 3.17 and 32768 x 4096 13.1 against 13.0; both bodies in one kernel,
+// behind a branch, 7.36, 3.24 and 13.5.  Two code objects leave one entry point
+// name to both.
+#ifdef AXH_WIDE_ONE_PASS
+constexpr bool kOnePassWide = true;
+#define AXH_ONE_PASS_BOUNDS __launch_bounds__(768)
+#else
+constexpr bool kOnePassWide = false;
+#define AXH_ONE_PASS_BOUNDS __launch_bounds__(512)
+#endif
+
 struct RowsArgs {
   uint32_t n_rows;
   uint32_t units_per_row; // superblocks (Q4_K) or blocks (Q4_0) per row
   uint32_t tile_units;    // units staged in LDS per tile (multiple of the wave step)
-  uint32_t pad;
+  uint32_t pad;           // wide one-pass kernels: waves per workgroup
 };
 
 struct CountArgs {
@@ -308,8 +326,10 @@ __device__ __forceinline__ void q4k_matvec_body(const uint8_t *__restrict__ q,
                                                 a.tile_units, blockIdx.x, axh_lds_dyn);          \
   }
 
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q4K_MATVEC_TILED(1, 4, 2)
 AXH_Q4K_MATVEC_TILED(2, 8, 2)
+#endif // AXH_WIDE_ONE_PASS
 
 // ---------------------------------------------------------------------------
 // Persistent Q4_K matvec for rows that fit one LDS tile (<= 128 superblocks).
@@ -853,7 +873,7 @@ __device__ __forceinline__ void q4k_matvec_flat(const uint8_t *__restrict__ q,
 // instances for rows of up to 16 superblocks are (axh_q5k_matvec_one_i{NIT},
 // see the runtime's Q5_K kernel choice).
 //
-// nw (8 to 12; 0: 8): the waves of the launch, 2 * nw rows per workgroup.  The
+// nw: the waves of a wide launch (9 to 12), 2 * nw rows per workgroup.  The
 // waves past the eighth stage the start of the next chunk, the values that it is
 // staged with an iteration later, before any wave reads it (a guard around
 // their loads and stores measured slower: Q4_K 8192 x 5376 with 8 waves 7.97 us
@@ -914,7 +934,8 @@ __device__ __forceinline__ void q4k_matvec_one(const uint8_t *__restrict__ q,
   // the first and of the second matrix, one row per lane slot, so the pair's
   // loads go through one wave-uniform resource each; W is the pair index.
   static_assert(!(kPair && kDual), "one pairing of gate and up rows");
-  const uint32_t W = kPair ? (blockIdx.x * NW + wave) >> 1 : blockIdx.x * (nw ? nw : 8u) + wave;
+  const uint32_t W = kPair ? (blockIdx.x * NW + wave) >> 1
+                           : blockIdx.x * (kOnePassWide ? nw : (uint32_t)NW) + wave;
   const bool mine = W < (n_rows + 1u) >> 1; // this wave has a pair of rows
   static_assert(!(kQ40 && (kDual || kQ5)), "Q4_0 rows are a layout of their own");
   // kQ40: nsb is the row's Q4_0 block count, read as octets of 8 blocks.
@@ -996,13 +1017,13 @@ __device__ __forceinline__ void q4k_matvec_one(const uint8_t *__restrict__ q,
 }
 
 #define AXH_Q4K_MATVEC_ONE(NIT)                                                                  \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q4k_matvec_one_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,      \
                                 float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn, a.pad);              \
   }                                                                                              \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q4k_matvec_onex_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
@@ -1026,14 +1047,14 @@ AXH_Q4K_MATVEC_ONE(15)
 AXH_Q4K_MATVEC_ONE(16)
 
 #define AXH_Q5K_MATVEC_ONE(NIT)                                                                  \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q5k_matvec_one_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,      \
                                 float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT, false, true>(q, q, x, y, a.n_rows, a.units_per_row, axh_lds_dyn, a.pad); \
   }
 #define AXH_Q5K_MATVEC_ONEP(NIT)                                                                 \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q5k_matvec_onep_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;        \
     extern __shared__ float axh_lds_dyn[];                                                       \
@@ -1056,7 +1077,7 @@ AXH_Q5K_MATVEC_ONE(8)
 AXH_Q5K_MATVEC_ONEP(8)
 
 #define AXH_Q4K_MATVEC_ONEP(NIT)                                                                 \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q4k_matvec_onep_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK; \
     extern __shared__ float axh_lds_dyn[];                                                       \
@@ -1416,6 +1437,7 @@ __device__ __forceinline__ void q6k_matvec_flat(const uint8_t *__restrict__ q,
                                                          a.units_per_row, axh_lds_dyn);          \
   }
 
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q5K_MATVEC_FLAT(1, 4, 2, 1)
 AXH_Q5K_MATVEC_FLAT(1, 4, 1, 1)
 AXH_Q5K_MATVEC_FLAT(1, 8, 1, 1)
@@ -1432,6 +1454,7 @@ AXH_Q6K_MATVEC_FLAT(1, 4, 4, 1)
 AXH_Q6K_MATVEC_FLAT(2, 4, 2, 1)
 AXH_Q6K_MATVEC_FLAT(1, 4, 2, 2)
 AXH_Q6K_MATVEC_FLAT(1, 8, 2, 2)
+#endif // AXH_WIDE_ONE_PASS
 
 // x chunk j of the Q6_K one-pass kernel: superblocks [8j, 8j + 8), float4 f
 // = 512j + tid + i*NT, staged with the mapping and layout of q6k_stage_xc.
@@ -1459,8 +1482,8 @@ __device__ __forceinline__ void q6k_stage_chunk(float *xs, float *ss, uint32_t t
 }
 
 // Q6_K one pass, one pair of rows per wave (axh_q6k_matvec_one_i{NIT}): rows
-// of 8 * (NIT - 1) < nsb <= 8 * NIT superblocks, 8 to 12 waves per workgroup
-// (nw), wave W takes rows 2W and 2W + 1, all workgroups launched.  The
+// of 8 * (NIT - 1) < nsb <= 8 * NIT superblocks, 8 waves per workgroup (wide:
+// nw, 9 to 12), wave W takes rows 2W and 2W + 1, all workgroups launched.  The
 // Q4_K one-pass order (q4k_matvec_one) with the Q6_K loads and decode of the
 // persistent kernel, so its output equals the persistent kernel's bit for
 // bit: x staged chunk by chunk (8 superblocks, 8 KiB) with the next
@@ -1480,7 +1503,7 @@ __device__ __forceinline__ void q6k_matvec_one(const uint8_t *__restrict__ q,
   const uint32_t lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t G = lane >> 2, half = G >> 3, s = G & 7u, c = lane & 3u;
-  const uint32_t W = blockIdx.x * (nw ? nw : 8u) + wave;
+  const uint32_t W = blockIdx.x * (kOnePassWide ? nw : (uint32_t)NW) + wave;
   const bool mine = W < (n_rows + 1u) >> 1; // this wave has a pair of rows
   // The host guarantees n_rows * row_bytes < 2^32 for this kernel.
   const uint32_t row_bytes = nsb * kQ6kSbBytes;
@@ -1512,7 +1535,7 @@ __device__ __forceinline__ void q6k_matvec_one(const uint8_t *__restrict__ q,
 }
 
 #define AXH_Q6K_MATVEC_ONE(NIT, XD, TAG)                                                         \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q6k_matvec_one##TAG##_i##NIT(const uint8_t *__restrict__ q,                            \
                                        const float *__restrict__ x, float *__restrict__ y,       \
                                        AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;                         \
@@ -1580,6 +1603,7 @@ AXH_Q6K_MATVEC_ONE(8, 2, p)
     q4k_matvec_one<NIT, false, Q5, true, 1, Q40, true>(qg, qu, x, y, a.n_rows,                   \
                                                        a.units_per_row, axh_lds_dyn);           \
   }
+#ifndef AXH_WIDE_ONE_PASS
 AXH_GATE_UP_ONE(q4k, false, false, 1)
 AXH_GATE_UP_ONE(q4_0, false, true, 1)
 AXH_GATE_UP_ONE(q5k, true, false, 1)
@@ -1656,6 +1680,7 @@ AXH_Q4K_MATVEC_FLAT_X2(1, 4, 2, 0)
 AXH_Q4K_MATVEC_FLAT_X2(1, 4, 4, 0)
 AXH_Q4K_MATVEC_FLAT_X2(2, 4, 2, 0)
 AXH_Q4K_MATVEC_FLAT_X2(2, 4, 4, 0)
+#endif // AXH_WIDE_ONE_PASS
 
 // ---------------------------------------------------------------------------
 // Column-slice Q4_K matvec: x held in VGPRs, rows streamed in batches.
@@ -1917,9 +1942,11 @@ __device__ __forceinline__ void q4k_matvec_wg(const uint8_t *__restrict__ q,
     q4k_matvec_wg<NW, XP, RB>(q, x, y, a.n_rows, a.units_per_row, axh_wg_dyn);                   \
   }
 
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q4K_MATVEC_WG(8, 2, 1)
 AXH_Q4K_MATVEC_WG(8, 2, 2)
 AXH_Q4K_MATVEC_WG(8, 2, 4)
+#endif // AXH_WIDE_ONE_PASS
 
 // ---------------------------------------------------------------------------
 // Split-K for few long rows (fewer than 32 rows of 64..256 superblocks that
@@ -2032,7 +2059,9 @@ __device__ __forceinline__ void q4k_matvec_sk(const uint8_t *__restrict__ q,
     q4k_matvec_sk<SPW>(q, x, y, ws, a.n_rows, a.units_per_row);                                  \
   }
 
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q4K_MATVEC_SK(16)
+#endif // AXH_WIDE_ONE_PASS
 
 #define AXH_Q4K_MATVEC_COLS(RB, NW, NT, XF)                                                       \
   extern "C" __global__ void __launch_bounds__(NW * 64)                                          \
@@ -2043,6 +2072,7 @@ AXH_Q4K_MATVEC_SK(16)
     q4k_matvec_cols<RB, NW, NT != 0, XF != 0>(q, x, y, a.n_rows, a.units_per_row, red);         \
   }
 
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q4K_MATVEC_COLS(4, 1, 0, 1)
 AXH_Q4K_MATVEC_COLS(4, 2, 0, 1)
 AXH_Q4K_MATVEC_COLS(4, 3, 0, 1)
@@ -2125,6 +2155,7 @@ extern "C" __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per
   const float r = wave_sum(acc);
   if (lane == 0) y[0] = r;
 }
+#endif // AXH_WIDE_ONE_PASS
 
 // ===========================================================================
 // Q4_0 matvec
@@ -2374,7 +2405,9 @@ __device__ __forceinline__ void q4_0_matvec_cols(const uint8_t *__restrict__ q,
     q4_0_matvec_cols<RB>(q, x, y, a.n_rows, a.units_per_row);                                    \
   }
 
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q4_0_MATVEC_COLS(1)
+#endif // AXH_WIDE_ONE_PASS
 
 #define AXH_Q4_0_MATVEC(RPW, NW)                                                                 \
   extern "C" __global__ void __launch_bounds__(NW * 64)                                          \
@@ -2386,10 +2419,12 @@ AXH_Q4_0_MATVEC_COLS(1)
                               axh_lds_dyn);                                                      \
   }
 
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q4_0_MATVEC(1, 1)
 AXH_Q4_0_MATVEC(1, 4)
 AXH_Q4_0_MATVEC(2, 4)
 AXH_Q4_0_MATVEC(4, 4)
+#endif // AXH_WIDE_ONE_PASS
 
 // Q4_0 through the Q4_K persistent and one-pass kernels (kQ40: octets of 8
 // blocks in place of superblocks, 64 blocks per iteration).
@@ -2406,6 +2441,7 @@ AXH_Q4_0_MATVEC(4, 4)
     q4k_matvec_flat<RPW, NW, PF, false, XP, false, false, true>(q, q, x, y, a.n_rows,            \
                                                                 a.units_per_row, axh_lds_dyn);   \
   }
+#ifndef AXH_WIDE_ONE_PASS
 AXH_Q4_0_MATVEC_FLAT(1, 4, 1, 1)
 AXH_Q4_0_MATVEC_FLAT(1, 8, 1, 1)
 AXH_Q4_0_MATVEC_FLAT(2, 4, 1, 1)
@@ -2413,19 +2449,20 @@ AXH_Q4_0_MATVEC_FLAT(2, 8, 1, 1)
 AXH_Q4_0_MATVEC_FLAT(1, 8, 2, 1)
 AXH_Q4_0_MATVEC_FLAT(2, 4, 2, 2)
 AXH_Q4_0_MATVEC_FLAT(1, 16, 2, 1)
+#endif // AXH_WIDE_ONE_PASS
 
 // axh_q4_0_matvec_one{,x,p}_i{NIT}: one workgroup of 8 waves per 16 rows of
 // 64 * (NIT - 1) < nb <= 64 * NIT blocks (x chunk by chunk, x whole, x two
 // chunks ahead).
 #define AXH_Q4_0_MATVEC_ONE(NIT)                                                                 \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q4_0_matvec_one_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,     \
                                  float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;        \
     extern __shared__ float axh_lds_dyn[];                                                       \
     q4k_matvec_one<NIT, false, false, false, 1, true>(q, q, x, y, a.n_rows, a.units_per_row,     \
                                                       axh_lds_dyn, a.pad);                       \
   }                                                                                              \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q4_0_matvec_onex_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,    \
                                   float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;       \
     extern __shared__ float axh_lds_dyn[];                                                       \
@@ -2433,7 +2470,7 @@ AXH_Q4_0_MATVEC_FLAT(1, 16, 2, 1)
                                                      axh_lds_dyn, a.pad);                        \
   }
 #define AXH_Q4_0_MATVEC_ONEP(NIT)                                                                \
-  extern "C" __global__ void __launch_bounds__(768)                                              \
+  extern "C" __global__ void AXH_ONE_PASS_BOUNDS                                                 \
       axh_q4_0_matvec_onep_i##NIT(const uint8_t *__restrict__ q, const float *__restrict__ x,    \
                                   float *__restrict__ y, AXH_ROWS_ARGS) { AXH_ROWS_UNPACK;       \
     extern __shared__ float axh_lds_dyn[];                                                       \
@@ -2471,6 +2508,7 @@ AXH_Q4_0_MATVEC_ONEP(14)
 AXH_Q4_0_MATVEC_ONEP(15)
 AXH_Q4_0_MATVEC_ONEP(16)
 
+#ifndef AXH_WIDE_ONE_PASS
 // Reference-compatible entry point for examples/q4_0_dequant_matvec.axc
 // (bindings q=0, x=1, y=2; push constant n_blocks: u32 @0; 1x1x1 of 64).
 // As q4km_dequant_matvec: x straight to registers.  Lane 4i + t takes dword t
@@ -2813,3 +2851,5 @@ extern "C" __global__ void __launch_bounds__(64) axh_spin(uint32_t *__restrict__
   for (uint32_t i = 0; i < a.n_units; ++i) __builtin_amdgcn_s_sleep(127);
   if (threadIdx.x == 0 && blockIdx.x == 0) out[0] = a.n_units;
 }
+
+#endif // AXH_WIDE_ONE_PASS

@@ -12,6 +12,8 @@
 // Code objects embedded by axh_embed.S (.incbin of the gfx950 ELFs).
 extern "C" const unsigned char axh_q4_matvec_co_begin[];
 extern "C" const unsigned char axh_q4_matvec_co_end[];
+extern "C" const unsigned char axh_q4_matvec_wide_co_begin[];
+extern "C" const unsigned char axh_q4_matvec_wide_co_end[];
 extern "C" const unsigned char axh_q4_matmul_co_begin[];
 extern "C" const unsigned char axh_q4_matmul_co_end[];
 
@@ -128,7 +130,8 @@ constexpr uint32_t kQ4_0MaxTileB = 1024; // 1024 * 132 B = 132 KiB of LDS
 } // namespace
 
 bool is_builtin_code_object(const void *co, size_t bytes) {
-  const unsigned char *objs[2][2] = {{axh_q4_matvec_co_begin, axh_q4_matvec_co_end},
+  const unsigned char *objs[3][2] = {{axh_q4_matvec_co_begin, axh_q4_matvec_co_end},
+                                     {axh_q4_matvec_wide_co_begin, axh_q4_matvec_wide_co_end},
                                      {axh_q4_matmul_co_begin, axh_q4_matmul_co_end}};
   for (const auto &o : objs) {
     const size_t n = (size_t)(o[1] - o[0]);
@@ -166,6 +169,9 @@ axh_status builtin_kernel(axh_context *ctx, const char *entry, uint32_t n_buffer
   if (std::strncmp(entry, "axh_q4k_matmul_", 15) == 0) {
     co = axh_q4_matmul_co_begin;
     n = (size_t)(axh_q4_matmul_co_end - axh_q4_matmul_co_begin);
+  } else if (wg_x > 512u && std::strstr(entry, "_matvec_one")) {
+    co = axh_q4_matvec_wide_co_begin; // one-pass workgroups of 9 to 12 waves
+    n = (size_t)(axh_q4_matvec_wide_co_end - axh_q4_matvec_wide_co_begin);
   }
   axh_kernel *k = nullptr;
   axh_status s = axh_prepare_kernel(ctx, co, n, &plan, pc_bytes, entry, &k);
