@@ -457,7 +457,7 @@ static bool q4k_use_wg(uint32_t n_rows, uint32_t nsb) {
 }
 
 // One pass with one pair of rows per wave (axh_q4k_matvec_one_i{NIT}, NIT =
-// ceil(nsb / 8)): one 8-wave workgroup per 16 rows (9 to 12 waves over 4097 to
+// ceil(nsb / 8)): one 8-wave workgroup per 16 rows (9 to 12 waves over 4105 to
 // 6144 rows, see one_pass_waves), all launched, each
 // staging x for its own rows.  Faster than the persistent kernels from 32 up
 // to 32768 rows (A/B in one run: 4096 x 14336 8.1-8.4 vs 8.5-8.7 us, 4096 x
@@ -526,10 +526,18 @@ static bool q4k_tiled_few(uint32_t n_rows, uint32_t nsb) {
 // 6.54 -> 6.33; Q6_K x 5376 9.25 -> 8.00, 9.36 -> 8.34, 9.61 -> 9.14; Q4_0 x
 // 14336 11.9 -> 9.42, 12.2 -> 10.8, 13.8 -> 11.0.  With 14 and 16 waves two
 // workgroups of 8, whose barriers do not stop each other, are ahead (Q4_K 7168
-// x 5376 6.83 against 7.22, 8192 x 5376 7.11 against 8.32).
+// x 5376 6.83 against 7.22, 8192 x 5376 7.11 against 8.32).  So do 8 waves up to
+// kOneWavesMinRows, where the one workgroup past one per CU holds at most four
+// pairs of rows: 9 waves took, in times of 8 waves at 4097, 4102, 4104 | 4106,
+// 4112 rows, Q4_K x 14336 1.10 (8.92 us against 8.07), 1.02, 1.00 | 0.84, 0.82;
+// x 4096 1.08 (3.61 against 3.31), 1.07, 1.07 | 0.96, 0.95; Q5_K x 4096 1.08, 1.06, 1.05 |
+// 0.95, 0.93; Q6_K x 5120 1.05, 1.03, 1.02 | 0.94, 0.91; Q4_0 x 4096 1.10, 1.06,
+// 1.08 | 1.00, 0.96.
+constexpr uint32_t kOneWavesMinRows = 4105;
+
 static uint32_t one_pass_waves(uint32_t n_rows) {
   const uint32_t pairs = n_rows / 2u + n_rows % 2u, w = (pairs + 255u) / 256u;
-  return w > 8u && w <= 12u ? w : 8u;
+  return n_rows >= kOneWavesMinRows && w <= 12u ? w : 8u;
 }
 
 static bool use_one_pass(uint32_t n_rows, uint32_t nsb) {
@@ -1151,19 +1159,21 @@ constexpr uint32_t kQ6OneMinRows = 256, kQ6OneMaxRows = 4096, kQ6OneWavesMaxRows
 // 8192 x 10240 15.24 vs 15.71; 4096 x 14336 11.79 vs 11.52 stays persistent).
 // At 2048 rows the 4-wave persistent kernel stays ahead (Q5_K 2048 x 14336
 // 7.64 vs 9.18).
-// Over 4113-6144 rows one workgroup of 9 to 12 waves per CU (one_pass_waves) is
-// ahead for all of 17-64 superblocks: 4352, 4999 and 6144 rows, Q5_K x 5376
-// 7.18, 7.30, 7.83 vs 8.00, 8.08, 8.35, x 14336 13.6, 14.2, 15.2 vs 17.4, 17.3,
-// 17.3; Q6_K x 14336 14.5, 16.4, 17.5 vs 18.6, 18.8, 18.9.  Up to 4112 rows, one
-// 8-wave workgroup past one per CU, the persistent kernel stays: the tests name
-// it at 4097.
+// Over 4105-6144 rows (kOneWavesMinRows) one workgroup of 9 to 12 waves per CU
+// is ahead for all of 17-64 superblocks, and for Q6_K rows of up to 16: 4352,
+// 4999 and 6144 rows, Q5_K x 5376 7.18, 7.30, 7.83 vs 8.00, 8.08, 8.35, x 14336
+// 13.6, 14.2, 15.2 vs 17.4, 17.3, 17.3; Q6_K x 14336 14.5, 16.4, 17.5 vs 18.6,
+// 18.8, 18.9.  The line is where the 9 waves start to pay: with them, 4104 rows
+// (4097) Q5_K x 4352 6.15 vs 7.00 (6.14 vs 6.05), x 8192 7.83 vs 8.27 (7.83 vs
+// 7.56), x 14336 11.5 vs 13.4 (11.5 vs 13.1), Q6_K x 4096 5.46 vs 5.56 (5.42 vs
+// 5.49), x 14336 12.5 vs 13.8 (12.5 vs 13.4).
 constexpr uint32_t kKqOneLongMinRows = 2049, kQ5OneLongMaxRows = 4096, kQ6OneLongMaxRows = 8192;
 constexpr uint32_t kQ5OneLongMaxSb = 64, kQ6OneLongMaxSb = 40;
-constexpr uint32_t kKqOneWavesMinRows = 4113, kKqOneWavesMaxRows = 6144;
+constexpr uint32_t kKqOneWavesMaxRows = 6144;
 
 static bool kq_one_long(const KqFormat &f, uint32_t n_rows, uint32_t nsb) {
   const bool q5 = &f == &kQ5kFormat;
-  if (n_rows >= kKqOneWavesMinRows &&
+  if (n_rows >= kOneWavesMinRows &&
       (nsb > kKqOneMaxSb ? n_rows <= kKqOneWavesMaxRows && nsb <= kQ5OneLongMaxSb
                          : n_rows <= kQ6OneWavesMaxRows))
     return true;

@@ -228,7 +228,8 @@ void axh_event_destroy(axh_event *ev);
  * steps); with no hole set they run one pass for rows of up to 16
  * superblocks over 768-32768 rows (Q5_K) or 256-4096 rows (Q6_K), and for
  * 2049-4096 rows of up to 64 superblocks (Q5_K) or 2049-8192 rows of up to 40
- * (Q6_K), else the persistent family (4 waves with x staged whole for up to
+ * (Q6_K), for 4105-6144 rows of 17-64 superblocks (both) and 4105-5120 rows of
+ * up to 16 (Q6_K), else the persistent family (4 waves with x staged whole for up to
  * 2048 rows of 17-64 superblocks and for 14336 rows and more of 33-64). */
 enum {
     AXH_Q4K_FAMILY_DEFAULT = 0,

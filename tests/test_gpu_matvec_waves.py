@@ -1,4 +1,4 @@
-"""One-pass matvecs with 9 to 12 waves per workgroup (marked `gpu`): 4097 to
+"""One-pass matvecs with 9 to 12 waves per workgroup (marked `gpu`): 4105 to
 6144 rows, one workgroup per CU.
 
 A row's sum is formed by one half wave in the same order whatever the size of
@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 # the first and last row counts of a wave count and of the range, odd counts,
 # rows of 1, 8, 9 superblocks and more; Q4_0 units are blocks
 @pytest.mark.parametrize("fmt,rows,units", [
-    ("q4k", 4097, 1), ("q4k", 4609, 9), ("q4k", 6144, 25), ("q4k", 6145, 9), ("q4k", 5000, 16),
+    ("q4k", 4097, 1), ("q4k", 4104, 16), ("q4k", 4105, 16), ("q5k", 4105, 17), ("q6k", 4105, 2),
+    ("q4_0", 4105, 66), ("q4k", 4609, 9), ("q4k", 6144, 25), ("q4k", 6145, 9), ("q4k", 5000, 16),
     ("q5k", 4097, 8), ("q5k", 5119, 17), ("q5k", 6144, 33), ("q6k", 4098, 16), ("q6k", 5120, 3),
     ("q6k", 6143, 41), ("q4_0", 4097, 64), ("q4_0", 6144, 130)])
 def test_rows_equal_those_of_smaller_calls(ctx, axc, fmt, rows, units):
@@ -51,8 +52,8 @@ def test_rows_equal_those_of_smaller_calls(ctx, axc, fmt, rows, units):
 
 
 @pytest.mark.parametrize("fmt,rows,units,one", [
-    ("q5k", 4112, 17, False), ("q5k", 4113, 17, True), ("q5k", 6144, 64, True),
-    ("q5k", 6145, 17, False), ("q6k", 4112, 16, False), ("q6k", 4113, 16, True),
+    ("q5k", 4104, 17, False), ("q5k", 4105, 17, True), ("q5k", 6144, 64, True),
+    ("q5k", 6145, 17, False), ("q6k", 4104, 16, False), ("q6k", 4105, 16, True),
     ("q6k", 5121, 16, False), ("q6k", 6144, 41, True), ("q6k", 6145, 41, False)])
 def test_defaults(axc, fmt, rows, units, one):
     name = getattr(axc, fmt + "_matvec_kernel_name")(rows, units)
