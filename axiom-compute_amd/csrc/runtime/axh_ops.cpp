@@ -1736,8 +1736,16 @@ static MatmulLaunch matmul_launch_of(const MatmulVariant &v, uint32_t n_rows, ui
     // Past one 16-row block per CU, while one round of 32 x 32 tiles covers
     // the grid (4096 x 4096 x 64 9.1 us against 12.4, 4096 x 1024 x 64 6.1
     // against 10.4, 1024 x 4096 x 250 8.8 against 12.0, A/B in one run); not
-    // before (4096 x 4096 x 32 8.6 against 7.3).
-    if (groups(16, 32) > kMatmulCus && groups(32, 32) <= kMatmulCus) k_groups = 8;
+    // before (4096 x 4096 x 32 8.6 against 7.3).  With one column group (4097
+    // to 8192 rows, up to 32 columns) the first body reads X once for all of a
+    // CU's blocks, and the tiles are ahead only where their 8 K groups come out
+    // even: 5000 rows x 24 columns, K = 1024, 1536, 1792, 2048, 2304, 3072, 3840,
+    // 4096: 0.89, 1.00, 1.09, 0.90, 1.04, 1.17, 1.33, 1.14 times the first
+    // body's time (3072: 8.31 us against 6.99; weights rotated through 0.4 to
+    // 1 GB 0.87, 0.97, 1.06, 0.91, 1.03, 1.16, 1.33, 1.11).
+    if (groups(16, 32) > kMatmulCus && groups(32, 32) <= kMatmulCus &&
+        (batch > 32 || nsb <= 6 || nsb == 8))
+      k_groups = 8;
   } else if (v.kind == 5 && v.rt == 4 && v.nt == 1) {
     // 32 x 32 tiles dequantise half of what 64 x 16 do (4096 x 14336 x 64 22
     // us against 39), but half their columns are empty up to 16.

@@ -1,0 +1,51 @@
+"""Which body the batched matmul's kernels with two bodies run (marked `gpu`).
+
+A body forms every output from its row's weights and its column's activations
+in an order of its own, whatever the size of the grid, so an output equals,
+bit for bit, the same output of a smaller call that runs the same body, and
+differs in some last bits where the other body runs."""
+from __future__ import annotations
+
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+class _Data:
+    def __init__(self, ctx, rows, sb, batch):
+        self.ctx, self.sb = ctx, sb
+        q = O.gen_q4k_weights(rows + sb, rows * sb)
+        xh = O.gen_normal_f32(sb + batch, sb * 256 * batch).astype(np.float16)
+        self.q, self.x, self.y = (ctx.alloc(n) for n in (q.nbytes, xh.nbytes, rows * batch * 4))
+        ctx.upload(self.q, q)
+        ctx.upload(self.x, xh)
+
+    def run(self, axc, rows, batch, variant=None):
+        print(f"matmul body {rows}x{self.sb * 256} B={batch} "
+              f"{axc.q4k_matmul_kernel_name(rows, self.sb, batch, variant)}", flush=True)
+        sys.stdout.flush()
+        self.ctx.q4k_matmul(self.q, self.x, self.y, rows, self.sb, batch, variant)
+        self.ctx.synchronize()
+        y = np.frombuffer(self.ctx.download(self.y, rows * batch * 4), dtype=np.uint32)
+        return y.reshape(batch, rows).copy()
+
+    def close(self):
+        for b in (self.q, self.x, self.y):
+            b.close()
+
+
+# 4096 rows of up to 32 columns: one 16-row block per CU, the first body
+@pytest.mark.parametrize("rows,sb,batch,tiles", [
+    (4097, 6, 17, True), (5000, 7, 24, False), (5000, 8, 24, True), (5000, 9, 24, False),
+    (5000, 12, 24, False), (8192, 15, 17, False), (8192, 16, 32, False)])
+def test_streaming_rows_with_one_column_group(ctx, axc, rows, sb, batch, tiles):
+    assert axc.q4k_matmul_kernel_name(rows, sb, batch) == "axh_q4k_matmul_sr_w8_s2_n2"
+    d = _Data(ctx, rows, sb, batch)
+    whole, first = d.run(axc, rows, batch), d.run(axc, 4096, batch)
+    d.close()
+    assert np.array_equal(whole[:, :4096], first) == (not tiles)
