@@ -617,15 +617,22 @@ __device__ __forceinline__ void q4k_matmul_lk(const uint8_t *__restrict__ q,
   // loads, the burst filled the load unit's queue and held the waves: A/B in
   // one run at 4096 x 14336, B = 8 13.31 vs 12.39 us, B = 16 15.92 vs 15.32,
   // B = 32 23.21 vs 22.17; at the end of the step, B = 32 took 23.05).  The
-  // issue order is fixed, so the loads issued after X of chunk c are always
-  // the 3 * RT weight loads of its group and the XD - 1 groups in between:
-  // waiting for that many leaves the weights ahead in flight.
-  auto step = [&](uint32_t c, auto e_c) {
+  // issue order is fixed, so the loads issued after X of chunk c are the 3 * RT
+  // weight loads of its group and the XD - 1 groups in between: waiting for that
+  // many leaves the weights ahead in flight.  The steps after the last whole
+  // round issue X (zeros past the row) but no weights: nothing would read them,
+  // so the compiler drops them, and a wait that counted them let the last loads
+  // of X land after the barrier.
+  auto step = [&](uint32_t c, auto e_c, auto tail_c) {
     constexpr int e = decltype(e_c)::value;
+    constexpr bool tail = decltype(tail_c)::value;
     // own X of chunk c landed; after the barrier every wave's X of chunk c is
     // in LDS and chunk c - 1's X buffer is free
-    static_assert((XD - 1) * kPer + 3 * RT <= 63, "vmcnt holds 6 bits");
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((XD - 1) * kPer + 3 * RT) : "memory");
+    constexpr int kAfter = !tail    ? (XD - 1) * kPer + 3 * RT
+                           : e < XD ? 3 * RT + (XD - 1 - e) * kPer + e * kXL
+                                    : (XD - 1) * kXL;
+    static_assert(kAfter <= 63, "vmcnt holds 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kAfter) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     issue_x(c + (uint32_t)XD, std::integral_constant<int, (e + XD) % XR>{});
     __builtin_amdgcn_sched_barrier(0);
@@ -656,7 +663,7 @@ __device__ __forceinline__ void q4k_matmul_lk(const uint8_t *__restrict__ q,
         const half8_t ahi = __builtin_bit_cast(half8_t, make_uint4(h0, h1, h2, h3));
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, xf[t], acc[i], 0, 0, 0);
         acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, xf[t + 4], acc[i], 0, 0, 0);
-        if (4 * i + t == 2 * RT - 1) { // halfway
+        if (!tail && 4 * i + t == 2 * RT - 1) { // halfway
           __builtin_amdgcn_sched_barrier(0);
           issue_w(c + (uint32_t)WD, std::integral_constant<int, (e + WD) % WR>{});
           __builtin_amdgcn_sched_barrier(0);
@@ -684,29 +691,32 @@ __device__ __forceinline__ void q4k_matmul_lk(const uint8_t *__restrict__ q,
   // Whole rounds of WR chunks, then the rest: no step of the loop body is
   // conditional, so no load is left in flight on a path around the back edge
   // (which made the compiler wait for every load at the loop head).
-  auto round = [&](uint32_t c0, auto e_c, bool guard) {
+  auto round = [&](uint32_t c0, auto e_c, auto tail_c) {
     constexpr int e = decltype(e_c)::value;
-    if constexpr (e < WR)
-      if (!guard || c0 + (uint32_t)e < n_ch) step(c0 + (uint32_t)e, e_c);
+    constexpr bool tail = decltype(tail_c)::value;
+    if constexpr (e < WR - (tail ? 1 : 0))
+      if (!tail || c0 + (uint32_t)e < n_ch) step(c0 + (uint32_t)e, e_c, tail_c);
   };
+  using Whole = std::integral_constant<bool, false>;
+  using Tail = std::integral_constant<bool, true>;
   uint32_t c0 = 0;
   for (; c0 + (uint32_t)WR <= n_ch; c0 += (uint32_t)WR) {
-    round(c0, std::integral_constant<int, 0>{}, false);
-    round(c0, std::integral_constant<int, 1>{}, false);
-    round(c0, std::integral_constant<int, 2>{}, false);
-    round(c0, std::integral_constant<int, 3>{}, false);
-    round(c0, std::integral_constant<int, 4>{}, false);
-    round(c0, std::integral_constant<int, 5>{}, false);
-    round(c0, std::integral_constant<int, 6>{}, false);
-    round(c0, std::integral_constant<int, 7>{}, false);
+    round(c0, std::integral_constant<int, 0>{}, Whole{});
+    round(c0, std::integral_constant<int, 1>{}, Whole{});
+    round(c0, std::integral_constant<int, 2>{}, Whole{});
+    round(c0, std::integral_constant<int, 3>{}, Whole{});
+    round(c0, std::integral_constant<int, 4>{}, Whole{});
+    round(c0, std::integral_constant<int, 5>{}, Whole{});
+    round(c0, std::integral_constant<int, 6>{}, Whole{});
+    round(c0, std::integral_constant<int, 7>{}, Whole{});
   }
-  round(c0, std::integral_constant<int, 0>{}, true);
-  round(c0, std::integral_constant<int, 1>{}, true);
-  round(c0, std::integral_constant<int, 2>{}, true);
-  round(c0, std::integral_constant<int, 3>{}, true);
-  round(c0, std::integral_constant<int, 4>{}, true);
-  round(c0, std::integral_constant<int, 5>{}, true);
-  round(c0, std::integral_constant<int, 6>{}, true);
+  round(c0, std::integral_constant<int, 0>{}, Tail{});
+  round(c0, std::integral_constant<int, 1>{}, Tail{});
+  round(c0, std::integral_constant<int, 2>{}, Tail{});
+  round(c0, std::integral_constant<int, 3>{}, Tail{});
+  round(c0, std::integral_constant<int, 4>{}, Tail{});
+  round(c0, std::integral_constant<int, 5>{}, Tail{});
+  round(c0, std::integral_constant<int, 6>{}, Tail{});
   // every load (the ones past the last chunk too) has landed before the LDS
   // is reused and before the waves end
   f32x4_t *red = lds + XR * kSlot;

@@ -1,0 +1,80 @@
+"""The long-rows matmul kernels' waits, checked on the built code (no GPU needed).
+
+A wave loads X into LDS for every wave of its workgroup and passes a barrier
+once its own loads have landed, which it tells from the load counter: loads
+return in the order they were issued, so after `s_waitcnt vmcnt(n)` all but the
+last n have.  Whether n is right depends on which loads the compiler kept and
+where it put them, so it is checked on the instructions: at every barrier no
+more loads of X may be in flight than those of the chunks requested ahead of
+the one that is read next."""
+from __future__ import annotations
+
+import ctypes
+import re
+import shutil
+import subprocess
+
+import pytest
+
+OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+@pytest.fixture(scope="module")
+def kernels(axc, tmp_path_factory):
+    """name -> instructions of every kernel of the matmul code object."""
+    if not shutil.which(OBJDUMP):
+        pytest.skip("llvm-objdump is not installed")
+    lib = axc.load_library()
+    begin, end = (ctypes.addressof(ctypes.c_char.in_dll(lib, f"axh_q4_matmul_co_{n}"))
+                  for n in ("begin", "end"))
+    co = tmp_path_factory.mktemp("co") / "q4_matmul.co"
+    co.write_bytes(ctypes.string_at(begin, end - begin))
+    text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(co)], check=True, text=True,
+                          stdout=subprocess.PIPE).stdout
+    out: dict = {}
+    for line in text.splitlines():
+        if m := re.match(r"^[0-9a-f]+ <(\w+)>:", line):
+            out[m.group(1)] = body = []
+        elif line.startswith("\t"):
+            body.append(line.split("//")[0].strip())
+    return out
+
+
+def _barriers(body):
+    """(index, loads of X in flight, LDS reads in flight) at every barrier,
+    along the instructions in address order (prologue, one turn of the loop, the
+    steps after it: a branch back enters where the fall-through does)."""
+    loads, reads, out = [], 0, []
+    for i, ins in enumerate(body):
+        op = ins.split()[0]
+        if op.startswith("buffer_load"):
+            loads.append(ins.endswith("lds"))
+        elif op.startswith("ds_read"):
+            reads += 1
+        elif op == "s_waitcnt":
+            if m := re.search(r"vmcnt\((\d+)\)", ins):
+                n = int(m.group(1))
+                loads = loads[len(loads) - n:] if n and n < len(loads) else loads if n else []
+            if m := re.search(r"lgkmcnt\((\d+)\)", ins):
+                reads = min(reads, int(m.group(1)))
+        elif op == "s_barrier":
+            out.append((i, sum(loads), reads))
+    return out
+
+
+LK = [("axh_q4k_matmul_lk_c16_x1_w3", 16, 1), ("axh_q4k_matmul_lk_c16_x1_w3_r2", 16, 1),
+      ("axh_q4k_matmul_lk_c8_x1_w3", 8, 1), ("axh_q4k_matmul_lk_c8_x2_w2", 8, 2),
+      ("axh_q4k_matmul_lk_c8_x2_w2_r2", 8, 2), ("axh_q4k_matmul_lk_c4_x2_w2", 4, 2)]
+
+
+@pytest.mark.parametrize("name,cols,ahead", LK)
+def test_x_has_landed_at_every_barrier(kernels, name, cols, ahead):
+    at = _barriers(kernels[name])
+    assert len(at) >= ahead + 3  # the steps of a round, those after it, and the sum
+    per_chunk = cols * 4 // 8  # loads of X per wave and chunk
+    for i, in_flight, _ in at:
+        assert in_flight <= (ahead - 1) * per_chunk, (name, i)
+
+
+def test_every_long_rows_kernel_is_listed(kernels):
+    assert {n for n in kernels if "_lk_" in n} == {n for n, _, _ in LK}
