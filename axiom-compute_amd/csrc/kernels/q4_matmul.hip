@@ -626,13 +626,14 @@ __device__ __forceinline__ void q4k_matmul_lk(const uint8_t *__restrict__ q,
   auto step = [&](uint32_t c, auto e_c, auto tail_c) {
     constexpr int e = decltype(e_c)::value;
     constexpr bool tail = decltype(tail_c)::value;
-    // own X of chunk c landed; after the barrier every wave's X of chunk c is
-    // in LDS and chunk c - 1's X buffer is free
+    // own X of chunk c landed, and chunk c - 1's fragments are in registers;
+    // after the barrier every wave's X of chunk c is in LDS and chunk c - 1's X
+    // buffer is free
     constexpr int kAfter = !tail    ? (XD - 1) * kPer + 3 * RT
                            : e < XD ? 3 * RT + (XD - 1 - e) * kPer + e * kXL
                                     : (XD - 1) * kXL;
     static_assert(kAfter <= 63, "vmcnt holds 6 bits");
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kAfter) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kAfter) : "memory");
     __builtin_amdgcn_sched_barrier(0);
     issue_x(c + (uint32_t)XD, std::integral_constant<int, (e + XD) % XR>{});
     __builtin_amdgcn_sched_barrier(0);

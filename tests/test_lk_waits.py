@@ -76,5 +76,12 @@ def test_x_has_landed_at_every_barrier(kernels, name, cols, ahead):
         assert in_flight <= (ahead - 1) * per_chunk, (name, i)
 
 
+@pytest.mark.parametrize("name,cols,ahead", LK)
+def test_x_is_read_before_its_buffer_is_refilled(kernels, name, cols, ahead):
+    """The loads after a barrier refill the buffer read before it."""
+    for i, _, reads in _barriers(kernels[name]):
+        assert reads == 0, (name, i)
+
+
 def test_every_long_rows_kernel_is_listed(kernels):
     assert {n for n in kernels if "_lk_" in n} == {n for n, _, _ in LK}
