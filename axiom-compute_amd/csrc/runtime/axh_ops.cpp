@@ -49,7 +49,8 @@ struct MatmulArgs {
 //                       flight.  r4 with n2, n4 p2 and n8 p2 (from 8 superblocks) and kind
 //                       8's r1 (from 4 at W = 4) run the wide-K-step body of 8 waves
 //                       (matmul_wide); n1 past 16 columns and kind 7's _n2 between one and
-//                       two blocks per CU its 32 x 32 form (matmul_launch_of).
+//                       two blocks per CU its 32 x 32 form, where that is ahead
+//                       (matmul_launch_of).
 //   kind 7 (streaming rows) axh_q4k_matmul_sr_w{W}_s2[_n2|_h]: persistent, one workgroup per
 //                       CU over 16-row blocks, K <= 4096 (pf 2: 8-column groups).
 //   kind 8 (32x32 tiles) axh_q4k_matmul_rm_w{W}_r{RT}_p4: W waves of RT 32-row MFMA tiles
@@ -1748,8 +1749,16 @@ static MatmulLaunch matmul_launch_of(const MatmulVariant &v, uint32_t n_rows, ui
       k_groups = 8;
   } else if (v.kind == 5 && v.rt == 4 && v.nt == 1) {
     // 32 x 32 tiles dequantise half of what 64 x 16 do (4096 x 14336 x 64 22
-    // us against 39), but half their columns are empty up to 16.
-    if (batch > 16) k_groups = 8;
+    // us against 39), but half their columns are empty up to 16, rows of fewer
+    // superblocks than K groups leave groups idle (one round of tiles, nsb = 1
+    // to 8: 1.36, 1.20, 1.21, 1.07, 1.08, 0.99, 0.99, 0.77 times as long), and
+    // a CU holds one of them, of the 64 x 16 tiles two: in several rounds they
+    // are ahead from 16 superblocks (0.83 to 0.88; 1.05 at 8 to 12), or from 32
+    // (0.75) where the last 16 columns are empty (48 columns: 1.2 at 21).
+    const bool half_empty = (batch - 1u) % 32u < 16u;
+    if (batch > 16 && nsb >= 8 &&
+        (groups(32, 32) <= kMatmulCus || nsb >= (half_empty ? 32u : 16u)))
+      k_groups = 8;
     l.threads = 512; // the kernel's; four of the waves end at once
   }
   if (k_groups == 8) {

@@ -467,8 +467,8 @@ typedef struct axh_q4_matmul_variant {
                                      says: rows or parts of K for each wave */
     uint32_t col_tiles;           /* 16-column MFMA tiles per workgroup (kind 8: 8;
                                      kind 9: 4-column groups, 1, 2 or 4; kind 5 with
-                                     1: 64 rows x 16 columns up to 16 columns, 32 x
-                                     32 beyond) */
+                                     1: 64 rows x 16 columns, or past 16 columns 32 x
+                                     32 where those are ahead) */
     uint32_t prefetch;            /* K steps in flight (kinds 3, 7; kind 7 prefetch 2:
                                      8-column groups), LDS ring depth (5, 8: 4; the
                                      main forms have their own), X

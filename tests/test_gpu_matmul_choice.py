@@ -39,6 +39,19 @@ class _Data:
             b.close()
 
 
+# 16 columns: 64 x 16 tiles, the first body of the one-column-tile kernel
+@pytest.mark.parametrize("rows,sb,batch,tiles", [
+    (300, 1, 48, False), (300, 7, 64, False), (300, 8, 33, True),      # one round of 32 x 32
+    (8224, 7, 17, False), (8224, 12, 64, False), (8224, 15, 32, False),  # more than one
+    (8224, 16, 32, True), (8224, 16, 48, False), (4128, 31, 48, False), (4128, 32, 48, True)])
+def test_one_column_tile(ctx, axc, rows, sb, batch, tiles):
+    v = axc.MatmulVariant(5, 4, 1, 3, 4)
+    d = _Data(ctx, rows, sb, batch)
+    whole, first = d.run(axc, rows, batch, v), d.run(axc, rows, 16, v)
+    d.close()
+    assert np.array_equal(whole[:16], first) == (not tiles)
+
+
 # 4096 rows of up to 32 columns: one 16-row block per CU, the first body
 @pytest.mark.parametrize("rows,sb,batch,tiles", [
     (4097, 6, 17, True), (5000, 7, 24, False), (5000, 8, 24, True), (5000, 9, 24, False),
