@@ -1867,7 +1867,12 @@ static MatmulVariant q4k_matmul_default(uint32_t n_rows, uint32_t batch, uint32_
   // 64: 5000 x 11008 x 128 34.5 against 50.9 in two rounds of 64 x 32.  Then 64
   // x 128 (8192 x 8192 x 256 46 us in one round, against 52 as four-wave
   // tiles), or the widest tile the columns fill.
+  // Rows of fewer than 8 superblocks run the narrow-step bodies, whose 64 x 16
+  // tiles come first where they fit: 5000 x 1024 x 33 5.57 us against 5.90 as
+  // 64 x 32, 4097 x 1792 x 40 7.88 against 8.19, 3000 x 512 x 77 4.33 against
+  // 4.67.
   if (batch > 16 && groups(32, 32) <= kMatmulCus) return {5, 4, 1, 3, 4};
+  if (nsb < 8 && groups(64, 16) <= kMatmulCus) return {5, 4, 1, 3, 4};
   if (batch <= 8) return {5, 4, 1, 3, 4}; // 64 x 16 (14336 x 14336 x 8 40 us)
   // 11008 x 11008 x 9 to 16 28 us in 64 x 32 tiles, 30 to 31.5 in 64 x 16
   uint32_t nt = 2;

@@ -52,6 +52,21 @@ def test_one_column_tile(ctx, axc, rows, sb, batch, tiles):
     assert np.array_equal(whole[:16], first) == (not tiles)
 
 
+# rows of few superblocks: 64 x 16 tiles while one round of them covers the grid
+@pytest.mark.parametrize("rows,sb,batch,kernel", [
+    (4097, 7, 48, "kx_r4_n1_k4_p3"), (4097, 8, 48, "kx_r4_n2_k4_p2"),
+    (5440, 1, 48, "kx_r4_n1_k4_p3"), (5441, 1, 48, "kx_r4_n2_k4_p2_short"),
+    (3264, 4, 77, "kx_r4_n1_k4_p3"), (3265, 4, 77, "kx_r4_n2_k4_p2_short")])
+def test_few_superblocks(ctx, axc, rows, sb, batch, kernel):
+    assert axc.q4k_matmul_kernel_name(rows, sb, batch) == "axh_q4k_matmul_" + kernel
+    d = _Data(ctx, rows, sb, batch)
+    whole = d.run(axc, rows, batch)
+    first = d.run(axc, rows, 16, axc.MatmulVariant(5, 4, 1, 3, 4))
+    d.close()
+    # the narrow-step tiles of every width split and sum K alike
+    assert np.array_equal(whole[:16], first) == (sb < 8)
+
+
 # 4096 rows of up to 32 columns: one 16-row block per CU, the first body
 @pytest.mark.parametrize("rows,sb,batch,tiles", [
     (4097, 6, 17, True), (5000, 7, 24, False), (5000, 8, 24, True), (5000, 9, 24, False),
