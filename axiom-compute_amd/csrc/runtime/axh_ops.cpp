@@ -1705,13 +1705,28 @@ constexpr uint64_t kMatmulFill = 160;
 // against 8.6, 2048 9.2 against 8.9, 4096 15.2 against 13.3, 14080 43.8 against
 // 38.5; two rounds of 2: 12000 x 256 columns, K = 768 13.4 against 14.2, 1024
 // equal, 2304 27.4 against 24.9, 14080 135 against 111) go to the _short form
-// of the kernel.
-static bool matmul_wide(const MatmulVariant &v, uint32_t nsb) {
-  if (v.kind == 5) return v.rt == 4 && v.nt > 1 && !(v.nt == 4 && v.pf == 3) && nsb >= 8;
-  return v.kind == 8 && v.rt == 1 && (v.w == 8 || nsb >= 4);
+// of the kernel.  So do the 64 x 32 tiles with two superblocks in flight (n2
+// p2) in more than one round of them, up to kShortRoundsMaxSb superblocks: a CU
+// holds two workgroups of that form and one of the wide one (28672 x 96
+// columns, nsb = 8, 12, 16, 21, 32: 1.25, 1.16, 1.14, 1.06, 1.03 times as long
+// wide; 9000 x 64 1.18, 1.09, 1.06, 1.00, 0.94).
+constexpr uint32_t kShortRoundsMaxSb = 23;
+
+static bool matmul_has_wide(const MatmulVariant &v) {
+  if (v.kind == 5) return v.rt == 4 && v.nt > 1 && !(v.nt == 4 && v.pf == 3);
+  return v.kind == 8 && v.rt == 1;
 }
-static bool matmul_short(const MatmulVariant &v, uint32_t nsb) {
-  return !matmul_wide(v, nsb) && matmul_wide(v, UINT32_MAX);
+
+static bool matmul_wide(const MatmulVariant &v, uint32_t n_rows, uint32_t batch, uint32_t nsb) {
+  if (!matmul_has_wide(v)) return false;
+  if (v.kind == 8) return v.w == 8 || nsb >= 4;
+  const uint64_t tiles =
+      (uint64_t)((n_rows + 63u) / 64u) * ((batch + 16u * v.nt - 1u) / (16u * v.nt));
+  const bool two_per_cu = v.nt == 2 && v.pf == 2;
+  return nsb >= (two_per_cu && tiles > kMatmulCus ? kShortRoundsMaxSb + 1u : 8u);
+}
+static bool matmul_short(const MatmulVariant &v, uint32_t n_rows, uint32_t batch, uint32_t nsb) {
+  return matmul_has_wide(v) && !matmul_wide(v, n_rows, batch, nsb);
 }
 
 // What a matmul variant launches for a shape: outputs per workgroup, threads,
@@ -1731,7 +1746,7 @@ static MatmulLaunch matmul_launch_of(const MatmulVariant &v, uint32_t n_rows, ui
   l.cols = v.kind == 9 ? 4u * v.nt : (v.kind == 7 && v.pf == 2 ? 8u : 16u) * v.nt;
   l.threads = v.w * 64u;
   uint32_t k_groups = 0; // of the wide-K-step body's 8 waves
-  if (matmul_wide(v, nsb)) {
+  if (matmul_wide(v, n_rows, batch, nsb)) {
     k_groups = v.kind == 5 ? 4u : 8u / v.w;
   } else if (v.kind == 7 && v.nt == 2) {
     // Past one 16-row block per CU, while one round of 32 x 32 tiles covers
@@ -1947,10 +1962,10 @@ static axh_status plan_q4k_matmul(uint32_t n_rows, uint32_t sb_per_row, uint32_t
                       v.rt == 1 ? "_r1" : "");
       else if (v.kind == 5)
         std::snprintf(name, cap, "axh_q4k_matmul_kx_r%u_n%u_k%u_p%u%s", v.rt, v.nt, v.w, v.pf,
-                      matmul_short(v, sb_per_row) ? "_short" : "");
+                      matmul_short(v, n_rows, batch, sb_per_row) ? "_short" : "");
       else if (v.kind == 8)
         std::snprintf(name, cap, "axh_q4k_matmul_rm_w%u_r%u_p4%s", v.w, v.rt,
-                      matmul_short(v, sb_per_row) ? "_short" : "");
+                      matmul_short(v, n_rows, batch, sb_per_row) ? "_short" : "");
       else if (v.kind == 9) {
         if (sb_per_row >= kLkMaxSb)
           return fail(AXH_ERR_INVALID_ARGUMENT,

@@ -67,6 +67,21 @@ def test_few_superblocks(ctx, axc, rows, sb, batch, kernel):
     assert np.array_equal(whole[:16], first) == (sb < 8)
 
 
+# 64 x 32 tiles with two superblocks in flight: the narrow-step form, two to a CU,
+# for several rounds of few superblocks
+@pytest.mark.parametrize("rows,sb,batch,kernel", [
+    (8192, 8, 64, "kx_r4_n2_k4_p2"), (8193, 8, 64, "kx_r4_n2_k4_p2_short"),
+    (8193, 23, 33, "kx_r4_n2_k4_p2_short"), (8193, 24, 33, "kx_r4_n2_k4_p2"),
+    (8193, 7, 33, "kx_r4_n2_k4_p2_short")])
+def test_two_column_tiles_in_rounds(ctx, axc, rows, sb, batch, kernel):
+    v = axc.MatmulVariant(5, 4, 2, 2, 4)
+    assert axc.q4k_matmul_kernel_name(rows, sb, batch, v) == "axh_q4k_matmul_" + kernel
+    d = _Data(ctx, rows, sb, batch)
+    whole, narrow = d.run(axc, rows, batch, v), d.run(axc, rows, 16, axc.MatmulVariant(5, 4, 1, 3, 4))
+    d.close()
+    assert np.array_equal(whole[:16], narrow) == kernel.endswith("_short")
+
+
 # 4096 rows of up to 32 columns: one 16-row block per CU, the first body
 @pytest.mark.parametrize("rows,sb,batch,tiles", [
     (4097, 6, 17, True), (5000, 7, 24, False), (5000, 8, 24, True), (5000, 9, 24, False),
