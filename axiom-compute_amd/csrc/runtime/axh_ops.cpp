@@ -47,7 +47,7 @@ struct MatmulArgs {
 //                       workgroup, its W waves splitting K by 64-wide superblock chunks,
 //                       register A, operands through per-wave LDS rings, PF superblocks in
 //                       flight.  r4 with n2, n4 p2 and n8 p2 (from 8 superblocks) and kind
-//                       8's r1 (from 4 at W = 4) run the wide-K-step body of 8 waves
+//                       8's r1 (from 6 at W = 4) run the wide-K-step body of 8 waves
 //                       (matmul_wide); n1 past 16 columns and kind 7's _n2 between one and
 //                       two blocks per CU its 32 x 32 form, where that is ahead
 //                       (matmul_launch_of).
@@ -1703,9 +1703,11 @@ constexpr uint64_t kMatmulFill = 160;
 // in 4 or 2, and rows too short for that (fewer than two rounds of 4
 // superblocks: 4096 rows x 128 columns, K = 1536 7.7 us with the narrow steps
 // against 8.6, 2048 9.2 against 8.9, 4096 15.2 against 13.3, 14080 43.8 against
-// 38.5; two rounds of 2: 12000 x 256 columns, K = 768 13.4 against 14.2, 1024
-// equal, 2304 27.4 against 24.9, 14080 135 against 111) go to the _short form
-// of the kernel.  So do the 64 x 32 tiles with two superblocks in flight (n2
+// 38.5; three rounds of 2: 32768 x 128 columns, K = 1024 15.8 against 16.8, 1280
+// 18.3 against 19.0, 1536 1.01 times as long wide; 11008 x 256, K = 1024, 1280,
+// 1536, 2048: 1.04, 1.01, 0.98, 0.96; four where the grid is more than one round:
+// 28672 x 256, K = 1024, 1536, 2048: 1.14, 1.06, 1.02) go to the _short form of the
+// kernel.  So do the 64 x 32 tiles with two superblocks in flight (n2
 // p2) in more than one round of them, up to kShortRoundsMaxSb superblocks: a CU
 // holds two workgroups of that form and one of the wide one (28672 x 96
 // columns, nsb = 8, 12, 16, 21, 32: 1.25, 1.16, 1.14, 1.06, 1.03 times as long
@@ -1719,11 +1721,12 @@ static bool matmul_has_wide(const MatmulVariant &v) {
 
 static bool matmul_wide(const MatmulVariant &v, uint32_t n_rows, uint32_t batch, uint32_t nsb) {
   if (!matmul_has_wide(v)) return false;
-  if (v.kind == 8) return v.w == 8 || nsb >= 4;
-  const uint64_t tiles =
-      (uint64_t)((n_rows + 63u) / 64u) * ((batch + 16u * v.nt - 1u) / (16u * v.nt));
+  const uint32_t rows = v.kind == 8 ? 32u * v.w : 64u, cols = 16u * v.nt;
+  const bool rounds =
+      (uint64_t)((n_rows + rows - 1u) / rows) * ((batch + cols - 1u) / cols) > kMatmulCus;
+  if (v.kind == 8) return v.w == 8 || nsb >= (rounds ? 8u : 6u);
   const bool two_per_cu = v.nt == 2 && v.pf == 2;
-  return nsb >= (two_per_cu && tiles > kMatmulCus ? kShortRoundsMaxSb + 1u : 8u);
+  return nsb >= (two_per_cu && rounds ? kShortRoundsMaxSb + 1u : 8u);
 }
 static bool matmul_short(const MatmulVariant &v, uint32_t n_rows, uint32_t batch, uint32_t nsb) {
   return matmul_has_wide(v) && !matmul_wide(v, n_rows, batch, nsb);

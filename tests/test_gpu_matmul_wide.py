@@ -61,8 +61,8 @@ def test_tiles_and_k_groups_at_their_edges(ctx, axc, rows, sb, batch):
     (16385, 8, 64, "kx_r4_n4_k4_p2"),          # none fits one round: the widest filled
     (16385, 7, 65, "kx_r4_n8_k4_p2_short"),
     (16385, 8, 65, "kx_r4_n8_k4_p2"),
-    (32768, 3, 128, "rm_w4_r1_p4_short"),
-    (32768, 4, 128, "rm_w4_r1_p4"),
+    (32768, 5, 128, "rm_w4_r1_p4_short"),
+    (32768, 6, 128, "rm_w4_r1_p4"),
     (32769, 1, 128, "rm_w8_r1_p4"),
 ])
 def test_default_tiles(ctx, axc, rows, sb, batch, kernel):
@@ -74,7 +74,8 @@ def test_default_tiles(ctx, axc, rows, sb, batch, kernel):
 @pytest.mark.parametrize("rows,sb,variant,kernel", [
     (300, 7, (5, 4, 8, 2, 4), "kx_r4_n8_k4_p2_short"), (300, 8, (5, 4, 8, 2, 4), "kx_r4_n8_k4_p2"),
     (300, 7, (5, 4, 2, 2, 4), "kx_r4_n2_k4_p2_short"), (300, 8, (5, 4, 2, 2, 4), "kx_r4_n2_k4_p2"),
-    (300, 3, (8, 4, 8, 4, 1), "rm_w4_r1_p4_short"), (300, 4, (8, 4, 8, 4, 1), "rm_w4_r1_p4"),
+    (300, 5, (8, 4, 8, 4, 1), "rm_w4_r1_p4_short"), (300, 6, (8, 4, 8, 4, 1), "rm_w4_r1_p4"),
+    (16400, 7, (8, 4, 8, 4, 1), "rm_w4_r1_p4_short"), (16400, 8, (8, 4, 8, 4, 1), "rm_w4_r1_p4"),
 ])
 def test_short_and_wide_steps(ctx, axc, rows, sb, variant, kernel):
     v = axc.MatmulVariant(*variant)
