@@ -1694,9 +1694,9 @@ constexpr uint32_t kSrMaxSb = 16;
 // with the wide-K-step bodies (figures at the rules).
 constexpr uint64_t kMatmulCus = 256;
 // Workgroups of 128 rows x 128 columns that kind 8 needs, and kind 9 of its own
-// tiles, before a smaller tile fills the chip better: 5/8 of the CUs (4096 x
-// 4096 x 256: 64-row x 64-column tiles in 256 workgroups 21.5 us, kind 8 in 64
-// workgroups 37.6).
+// tiles, before a smaller tile fills the chip better (where one round holds it):
+// 5/8 of the CUs (4096 x 4096 x 256: 64-row x 64-column tiles in 256 workgroups
+// 21.5 us, kind 8 in 64 workgroups 37.6).
 constexpr uint64_t kMatmulFill = 160;
 
 // Whether a kind 5 or 8 variant runs the wide-K-step body: its 8 waves split K
@@ -1873,8 +1873,12 @@ static MatmulVariant q4k_matmul_default(uint32_t n_rows, uint32_t batch, uint32_
   // 4096 x 256 36.5 us, against 42 before they split K), then 256-row tiles
   // (28672 x 4096 x 256 67.6 us against 83.6 with 128-row tiles in two rounds,
   // 40960 x 4096 x 128 60.5 against 69, 18432 x 4096 x 256 62.2 against 66.3).
-  // Below the fill the K-split tiles are ahead (11008 x 4096 x 128).
-  if (batch >= 128 && groups(128, 128) >= kMatmulFill)
+  // Below the fill the K-split tiles are ahead (11008 x 4096 x 128), while 64 x
+  // 128 ones are one round: 8192 x 4096 x 256 25.8 us in 256 of them against
+  // 30.1, but 8193 rows 44.0 against 33.9, 9216 x 4096 x 256 41.5 against 30.5,
+  // 18432 x 4096 x 128 43.7 against 31.3, 4608 x 4096 x 512 41.5 against 31.0,
+  // 10112 x 14336 x 256 133 against 97, 9216 x 768 x 256 18.5 against 11.1.
+  if (batch >= 128 && (groups(128, 128) >= kMatmulFill || groups(64, 128) > kMatmulCus))
     return groups(128, 128) > kMatmulCus ? MatmulVariant{8, 8, 8, 4, 1}
                                          : MatmulVariant{8, 4, 8, 4, 1};
   // Kind 5 beyond: the narrowest of its tiles whose grid is one round, since a

@@ -61,6 +61,13 @@ def test_tiles_and_k_groups_at_their_edges(ctx, axc, rows, sb, batch):
     (16385, 8, 64, "kx_r4_n4_k4_p2"),          # none fits one round: the widest filled
     (16385, 7, 65, "kx_r4_n8_k4_p2_short"),
     (16385, 8, 65, "kx_r4_n8_k4_p2"),
+    (8192, 16, 256, "kx_r4_n8_k4_p2"),         # 128 x 2 of 64 x 128
+    (8193, 16, 256, "rm_w4_r1_p4"),            # 129 x 2: 65 x 2 of 128 x 128
+    (8193, 3, 256, "rm_w4_r1_p4_short"),
+    (16384, 9, 128, "kx_r4_n8_k4_p2"), (16385, 9, 128, "rm_w4_r1_p4"),
+    (16385, 9, 127, "kx_r4_n8_k4_p2"),
+    (20352, 9, 128, "rm_w4_r1_p4"),            # 159 of 128 x 128
+    (4608, 9, 512, "rm_w4_r1_p4"),
     (32768, 5, 128, "rm_w4_r1_p4_short"),
     (32768, 6, 128, "rm_w4_r1_p4"),
     (32769, 1, 128, "rm_w8_r1_p4"),
