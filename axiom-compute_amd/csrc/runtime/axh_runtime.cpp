@@ -550,14 +550,25 @@ static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_
     if (e != hipSuccess) return fail(AXH_ERR_MEMORY_MAP, hip_msg("hipHostMalloc", e));
     k->staging_bytes = want;
   }
-  // After an error copies may still be queued on the staging buffer: it is
-  // freed with the core, and the next dispatch takes a fresh one.
-  auto retire = [&](axh_status st) {
-    std::lock_guard<std::mutex> lk(core.staging_mu);
-    if (k->staging) core.retired_staging.push_back(k->staging);
-    k->staging = nullptr;
-    k->staging_bytes = 0;
+  // Waits for all of it.  A timeout leaves copies queued on the staging buffer:
+  // it is freed with the core, and the next dispatch takes a fresh one.
+  auto finish = [&]() {
+    const axh_status st = wait_stream(core, core.stream);
+    if (st == AXH_ERR_FENCE_TIMEOUT) {
+      std::lock_guard<std::mutex> lk(core.staging_mu);
+      core.retired_staging.push_back(k->staging);
+      k->staging = nullptr;
+      k->staging_bytes = 0;
+    }
     return st;
+  };
+  // An error in between leaves what was queued before it: once that is done the
+  // handle keeps its buffer, so a request that is refused every time costs
+  // nothing but itself.
+  auto drop = [&](axh_status st) {
+    const std::string msg = t_last_error;
+    finish();
+    return fail(st, msg);
   };
   auto copy_launch = [&](CopySegment *table, uint32_t segs, size_t largest) {
     if (segs == 0) return AXH_OK;
@@ -579,16 +590,16 @@ static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_
     } else {
       e = hipMemcpyAsync(k->pool[i], at, input_sizes[i], hipMemcpyHostToDevice, core.stream);
       if (e != hipSuccess)
-        return retire(fail(AXH_ERR_STAGING_COPY, "binding #" + std::to_string(i) +
-                                                     " (HostToDevice): " +
-                                                     hip_msg("hipMemcpyAsync", e)));
+        return drop(fail(AXH_ERR_STAGING_COPY, "binding #" + std::to_string(i) +
+                                                   " (HostToDevice): " +
+                                                   hip_msg("hipMemcpyAsync", e)));
     }
     at += staged_size(input_sizes[i]);
   }
   s = copy_launch(tin, segs, largest);
-  if (s != AXH_OK) return retire(s);
+  if (s != AXH_OK) return drop(s);
   s = launch_raw(k, workgroups, k->pool.data(), n, pc, pc_bytes, 0, core.stream);
-  if (s != AXH_OK) return retire(s);
+  if (s != AXH_OK) return drop(s);
   const uint8_t *out = at;
   segs = 0;
   largest = 0;
@@ -600,15 +611,15 @@ static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_
     } else {
       e = hipMemcpyAsync(at, k->pool[i], output_sizes[i], hipMemcpyDeviceToHost, core.stream);
       if (e != hipSuccess)
-        return retire(fail(AXH_ERR_READBACK, "readback of binding #" + std::to_string(i) +
-                                                 " failed: " + hip_msg("hipMemcpyAsync", e)));
+        return drop(fail(AXH_ERR_READBACK, "readback of binding #" + std::to_string(i) +
+                                               " failed: " + hip_msg("hipMemcpyAsync", e)));
     }
     at += staged_size(output_sizes[i]);
   }
   s = copy_launch(tout, segs, largest);
-  if (s != AXH_OK) return retire(s);
-  s = wait_stream(core, core.stream);
-  if (s != AXH_OK) return retire(s);
+  if (s != AXH_OK) return drop(s);
+  s = finish();
+  if (s != AXH_OK) return s;
   for (size_t i = 0; i < n; ++i) {
     if (output_sizes[i] == 0) continue;
     std::memcpy(outputs[i], out, output_sizes[i]);
