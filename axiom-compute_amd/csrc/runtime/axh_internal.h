@@ -26,6 +26,11 @@ struct LoadedModule {
   int refs = 0;
 };
 
+struct PinnedBuffer {
+  void *p = nullptr;
+  size_t bytes = 0;
+};
+
 // Device-side state shared by a context and every handle prepared on it, so
 // a handle may outlive the context that made it.
 struct Core {
@@ -46,6 +51,11 @@ struct Core {
 
   std::mutex event_mu;
   std::vector<hipEvent_t> idle_events; // kept between completion waits
+
+  // Pinned staging buffers of dispatch_handle between dispatches, the last used
+  // one at the end; bounded (kMaxIdlePinned, kMaxIdlePinnedBytes).
+  std::mutex pinned_mu;
+  std::vector<PinnedBuffer> idle_pinned;
 
   std::mutex cache_mu; // guards modules and kernels
   std::unordered_map<uint64_t, LoadedModule> modules;
@@ -74,8 +84,6 @@ struct axh_kernel {
   std::mutex mu;              // serialises dispatch_handle on this handle
   std::vector<void *> pool;   // per-binding device buffers
   std::vector<size_t> pool_bytes;
-  void *staging = nullptr; // pinned host memory of dispatch_handle (at most 32 MiB)
-  size_t staging_bytes = 0;
 };
 
 struct axh_context {

@@ -51,6 +51,7 @@ Core::~Core() {
   if (stream) hipStreamSynchronize(stream); // retired staging buffers may still be in use
   if (staging) hipHostFree(staging);
   for (void *p : retired_staging) hipHostFree(p);
+  for (const PinnedBuffer &b : idle_pinned) hipHostFree(b.p);
   for (hipEvent_t ev : idle_events) hipEventDestroy(ev);
   if (stream) hipStreamDestroy(stream);
 }
@@ -499,7 +500,6 @@ void axh_kernel_release(axh_kernel *k) {
     hipSetDevice(core->device);
     for (void *p : k->pool)
       if (p) hipFree(p);
-    if (k->staging) hipHostFree(k->staging);
     release_module(*core, k->module_hash);
   }
   delete k; // the last holder of `core` may free the device state here
@@ -512,7 +512,51 @@ uint64_t axh_kernel_pool_bytes(const axh_kernel *k, uint32_t binding) {
   return k->pool_bytes[binding];
 }
 
-// A binding's share of a handle's staging buffer (256-byte aligned).
+// Staging buffers are shared by the handles of a context: one that lives for a
+// single dispatch, or one of many, pins nothing of its own, and its release
+// frees no pinned memory (which can wait for the device).
+static constexpr size_t kMaxIdlePinned = 8;
+static constexpr size_t kMaxIdlePinnedBytes = 2 * kStagingChunk;
+
+// The smallest idle buffer of at least `bytes`, or a new one.
+static axh_status take_pinned(Core &core, size_t bytes, PinnedBuffer *out) {
+  {
+    std::lock_guard<std::mutex> lk(core.pinned_mu);
+    auto best = core.idle_pinned.end();
+    for (auto it = core.idle_pinned.begin(); it != core.idle_pinned.end(); ++it)
+      if (it->bytes >= bytes && (best == core.idle_pinned.end() || it->bytes < best->bytes))
+        best = it;
+    if (best != core.idle_pinned.end()) {
+      *out = *best;
+      core.idle_pinned.erase(best);
+      return AXH_OK;
+    }
+  }
+  const size_t want = round_up_pow2(bytes);
+  hipError_t e = hipHostMalloc(&out->p, want, hipHostMallocDefault);
+  if (e != hipSuccess) return fail(AXH_ERR_MEMORY_MAP, hip_msg("hipHostMalloc", e));
+  out->bytes = want;
+  return AXH_OK;
+}
+
+// Back to the idle ones; the ones unused for longest go past the bounds.
+static void give_pinned(Core &core, PinnedBuffer b) {
+  std::vector<PinnedBuffer> surplus;
+  {
+    std::lock_guard<std::mutex> lk(core.pinned_mu);
+    core.idle_pinned.push_back(b);
+    size_t total = 0;
+    for (const PinnedBuffer &i : core.idle_pinned) total += i.bytes;
+    while (core.idle_pinned.size() > kMaxIdlePinned || total > kMaxIdlePinnedBytes) {
+      surplus.push_back(core.idle_pinned.front());
+      total -= surplus.back().bytes;
+      core.idle_pinned.erase(core.idle_pinned.begin());
+    }
+  }
+  for (const PinnedBuffer &i : surplus) hipHostFree(i.p);
+}
+
+// A binding's share of a staging buffer (256-byte aligned).
 static size_t staged_size(size_t bytes) {
   return bytes > kStagingChunk ? kStagingChunk + 1 : (bytes + 255u) & ~size_t(255);
 }
@@ -528,42 +572,27 @@ struct CopySegment {
 static constexpr size_t kKernelCopyBytes = size_t(2) << 20;
 static constexpr uint32_t kCopyWgs = 64; // workgroups per segment
 
-// dispatch_handle's device work through the handle's staging buffer; k->mu is
-// held and the pool is sized.  The buffer holds the two segment tables, the
-// inputs and the outputs (`packed` bytes).
-static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
+// dispatch_handle's device work through a staging buffer; k->mu is held and the
+// pool is sized.  The buffer holds the two segment tables, the inputs and the
+// outputs.  *busy: copies may still be queued on it when this returns.
+static axh_status dispatch_staged(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
                                   const void *const *inputs, const size_t *input_sizes,
                                   const size_t *output_sizes, void *const *outputs, const void *pc,
-                                  size_t pc_bytes, size_t packed) {
+                                  size_t pc_bytes, void *staging, bool *busy) {
   Core &core = *ctx->core;
   const size_t n = k->access.size();
   axh_kernel *copy = nullptr;
   axh_status s = builtin_kernel(ctx, "axh_copy_segments", 1, 4, 256, &copy);
   if (s != AXH_OK) return s;
   hipError_t e = hipSuccess;
-  if (k->staging_bytes < packed) {
-    if (k->staging) hipHostFree(k->staging);
-    k->staging = nullptr;
-    k->staging_bytes = 0;
-    const size_t want = round_up_pow2(packed);
-    e = hipHostMalloc(&k->staging, want, hipHostMallocDefault);
-    if (e != hipSuccess) return fail(AXH_ERR_MEMORY_MAP, hip_msg("hipHostMalloc", e));
-    k->staging_bytes = want;
-  }
-  // Waits for all of it.  A timeout leaves copies queued on the staging buffer:
-  // it is freed with the core, and the next dispatch takes a fresh one.
+  // Waits for all of it; a timeout leaves copies queued on the staging buffer.
   auto finish = [&]() {
     const axh_status st = wait_stream(core, core.stream);
-    if (st == AXH_ERR_FENCE_TIMEOUT) {
-      std::lock_guard<std::mutex> lk(core.staging_mu);
-      core.retired_staging.push_back(k->staging);
-      k->staging = nullptr;
-      k->staging_bytes = 0;
-    }
+    *busy = st == AXH_ERR_FENCE_TIMEOUT;
     return st;
   };
   // An error in between leaves what was queued before it: once that is done the
-  // handle keeps its buffer, so a request that is refused every time costs
+  // buffer can be used again, so a request that is refused every time costs
   // nothing but itself.
   auto drop = [&](axh_status st) {
     const std::string msg = t_last_error;
@@ -577,8 +606,8 @@ static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_
     void *bufs[1] = {table};
     return launch_raw(copy, grid, bufs, 1, &segs, sizeof(segs), 0, core.stream);
   };
-  CopySegment *tin = static_cast<CopySegment *>(k->staging), *tout = tin + n;
-  uint8_t *at = static_cast<uint8_t *>(k->staging) + staged_size(2 * n * sizeof(CopySegment));
+  CopySegment *tin = static_cast<CopySegment *>(staging), *tout = tin + n;
+  uint8_t *at = static_cast<uint8_t *>(staging) + staged_size(2 * n * sizeof(CopySegment));
   uint32_t segs = 0;
   size_t largest = 0;
   for (size_t i = 0; i < n; ++i) {
@@ -626,6 +655,26 @@ static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_
     out += staged_size(output_sizes[i]);
   }
   return AXH_OK;
+}
+
+static axh_status dispatch_packed(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
+                                  const void *const *inputs, const size_t *input_sizes,
+                                  const size_t *output_sizes, void *const *outputs, const void *pc,
+                                  size_t pc_bytes, size_t packed) {
+  Core &core = *ctx->core;
+  PinnedBuffer b;
+  axh_status s = take_pinned(core, packed, &b);
+  if (s != AXH_OK) return s;
+  bool busy = false;
+  s = dispatch_staged(ctx, k, workgroups, inputs, input_sizes, output_sizes, outputs, pc, pc_bytes,
+                      b.p, &busy);
+  if (busy) { // freed with the core
+    std::lock_guard<std::mutex> lk(core.staging_mu);
+    core.retired_staging.push_back(b.p);
+  } else {
+    give_pinned(core, b);
+  }
+  return s;
 }
 
 axh_status axh_dispatch_handle(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
@@ -678,10 +727,9 @@ axh_status axh_dispatch_handle(axh_context *ctx, axh_kernel *k, const uint32_t w
     k->pool[i] = p;
     k->pool_bytes[i] = sz;
   }
-  // Requests up to kStagingChunk bytes go through the handle's own pinned
-  // buffer, inputs and outputs side by side: the copies and the launch are
-  // queued behind each other and waited for once.  Larger ones stage and wait
-  // for each binding by itself.
+  // Requests up to kStagingChunk bytes go through one pinned buffer, inputs and
+  // outputs side by side: the copies and the launch are queued behind each other
+  // and waited for once.  Larger ones stage and wait for each binding by itself.
   size_t packed = staged_size(2 * n * sizeof(CopySegment));
   for (size_t i = 0; i < n; ++i) {
     packed += staged_size(input_sizes[i]);

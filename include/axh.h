@@ -127,7 +127,12 @@ uint64_t axh_kernel_pool_bytes(const axh_kernel *k, uint32_t binding);
  * with the fence timeout and copies output_sizes[i] bytes of every binding
  * into outputs[i] (skipped when output_sizes[i] == 0).  Validation happens
  * before any device work (dispatch.rs:56-95).  Dispatches on one handle are
- * serialised; different handles may dispatch concurrently. */
+ * serialised; different handles may dispatch concurrently.  Requests of up to
+ * 32 MiB in all go through one pinned buffer each, taken from the context for
+ * the call: it keeps up to 8 of them and 64 MiB between calls, for all its
+ * handles, until it is destroyed (besides the one of up to 32 MiB that larger
+ * requests, uploads and downloads share).  A request that times out keeps its
+ * buffer until then. */
 axh_status axh_dispatch_handle(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
                                const void *const *inputs, const size_t *input_sizes,
                                size_t n_inputs, const size_t *output_sizes, size_t n_outputs,
@@ -150,7 +155,10 @@ axh_status axh_validate_request(const axh_binding_plan *plan, const uint32_t wor
 /* ---- resident buffers and asynchronous launch ------------------------------
  * The hot path: buffers stay in HBM between calls; launches are asynchronous
  * on `stream`.  Uploads/downloads go through the context's pinned staging
- * buffer with hipMemcpyAsync and return when the copy is complete. */
+ * buffer with hipMemcpyAsync and return when the copy is complete.  Every wait
+ * of this library for a stream (synchronize, uploads, downloads, dispatches)
+ * polls for its first 500 us without sleeping, then every 20 us: a waiting
+ * thread is busy for that long. */
 axh_status axh_buffer_alloc(axh_context *ctx, size_t bytes, void **device_ptr);
 axh_status axh_buffer_free(axh_context *ctx, void *device_ptr);
 axh_status axh_upload(axh_context *ctx, void *device_dst, const void *host_src, size_t bytes);

@@ -1,8 +1,9 @@
-"""dispatch_handle after requests that fail (marked `gpu`): what a handle and its
-context hold, and the next request on the same handle."""
+"""What dispatch_handle keeps, after requests that fail too (marked `gpu`): pinned
+memory of a handle and its context, and the next request on the same handle."""
 from __future__ import annotations
 
 import struct
+import threading
 
 import numpy as np
 import pytest
@@ -54,4 +55,79 @@ def test_refused_launches_keep_nothing(axc):
     assert _widen(ctx, good, h[:4096])
     good.release()
     bad.release()
+    ctx.close()
+
+
+def test_dispatch_after_a_timed_out_one(axc):
+    """The same handle, whose first request (a ~10 ms kernel) outlasted the 5 ms
+    timeout: its copies may still use the buffer that it was given."""
+    print("dispatch after a timeout", flush=True)
+    ctx = axc.HipContext.new_with_options(axc.HipContextOptions(fence_timeout_ms=5))
+    k = ctx.prepare_kernel(axc.builtin_code_object(), _plan(axc, 1, 4, 64), 4, "axh_spin")
+    for _ in range(2):
+        with pytest.raises(axc.DispatchError) as e:
+            ctx.dispatch_handle(k, (1, 1, 1), [b""], [4], struct.pack("<I", 3000))
+        assert e.value.variant == "FenceTimeout"
+        ctx.device_synchronize()  # unbounded wait: the bounded kernel ends by itself
+        for n in (10, 11):
+            out = ctx.dispatch_handle(k, (1, 1, 1), [b""], [4], struct.pack("<I", n))
+            assert struct.unpack("<I", out[0])[0] == n
+    k.release()
+    ctx.close()
+
+
+def test_handles_share_their_pinned_memory(axc):
+    """Eight live handles, each with a request of 8 MiB: one staging buffer of 16
+    MiB, not one for each (which a handle held for its life)."""
+    print("pinned memory of many handles", flush=True)
+    ctx = axc.HipContext.new()
+    h = np.random.default_rng(4).integers(0, 0x7C00, 4 << 20).astype(np.uint16)
+    modes = [axc.axh.ACCESS_READ_ONLY, axc.axh.ACCESS_READ_WRITE]
+    handles = [ctx.prepare_kernel(axc.builtin_code_object(),
+                                  axc.BindingPlan([a, b], 4, (wg, 1, 1)), 4, "axh_f16_widen")
+               for a in modes for b in modes for wg in (128, 256)]
+    assert len({k.cache_key for k in handles}) == 8
+
+    def request(k, n):
+        ctx.dispatch_handle(k, (1, 1, 1), [h[:n].tobytes(), b""], [0, 4], struct.pack("<I", 256))
+
+    for k in handles:
+        request(k, 16)
+    before = _address_space()
+    for k in handles:
+        request(k, h.size)
+    grown = _address_space() - before
+    print(f"  address space grew by {grown >> 20} MiB", flush=True)
+    assert grown < (8 * 8 + 8 * 16) << 20  # device buffers of 8 MiB, and less than eight of these
+    for k in handles:
+        k.release()
+    ctx.close()
+
+
+def test_concurrent_dispatches_use_buffers_of_their_own(axc):
+    print("concurrent dispatches", flush=True)
+    ctx = axc.HipContext.new()
+    errors = []
+
+    def work(seed):
+        try:
+            rng = np.random.default_rng(seed)
+            # a handle of this thread's own: another access list or launch size
+            mode = axc.axh.ACCESS_READ_ONLY if seed & 1 else axc.axh.ACCESS_READ_WRITE
+            k = ctx.prepare_kernel(axc.builtin_code_object(),
+                                   axc.BindingPlan([mode, axc.axh.ACCESS_READ_WRITE], 4,
+                                                   (256, 1, 1)), 4, "axh_f16_widen")
+            for _ in range(12):
+                n = int(rng.choice([100, 5000, 1 << 17, 3 << 19]))
+                assert _widen(ctx, k, rng.integers(0, 0x7C00, n).astype(np.uint16))
+            k.release()
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
     ctx.close()
