@@ -461,7 +461,15 @@ axh_status axh_q4_0_matvec_variant_at(uint32_t i, axh_q4_variant *out);
  * contiguous f16 activation vectors.  Y is batch x n_rows f32.  The reference
  * has no batched kernel (its matvec, examples/q4km_dequant_matvec.axc, is the
  * batch = 1 case with f32 weights); multi-row matmul is roadmap there
- * (ROADMAP.md:54-72).  q and x 16-byte aligned, each below 4 GiB. */
+ * (ROADMAP.md:54-72).  q and x 16-byte aligned, each below 4 GiB.
+ *
+ * A variant of zeros is the default.  Beside other fields a 0 takes the value
+ * that the default has for the shape, with two exceptions that do not follow
+ * the lines between the default's tiles: kind 8's waves_per_workgroup is 4, or
+ * 8 past 256 columns where 256-row tiles make 160 workgroups, and kind 5's
+ * col_tiles is what the columns fill (1, 2, 4 or 8), halved until 64-row tiles
+ * make 160 workgroups, with its prefetch.  So naming only the kind that the
+ * default has can select other tiles than the default. */
 typedef struct axh_q4_matmul_variant {
     uint32_t kind;                /* 3 K-split, 5 K-split tile, 7 streaming rows
                                      (K <= 4096), 8 32x32 tiles (128 columns per

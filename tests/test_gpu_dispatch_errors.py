@@ -98,7 +98,8 @@ def test_handles_share_their_pinned_memory(axc):
         request(k, h.size)
     grown = _address_space() - before
     print(f"  address space grew by {grown >> 20} MiB", flush=True)
-    assert grown < (8 * 8 + 8 * 16) << 20  # device buffers of 8 MiB, and less than eight of these
+    # eight device buffers of 8 MiB and one staging buffer: 85 MiB; 194 with eight of them
+    assert grown < 128 << 20
     for k in handles:
         k.release()
     ctx.close()
