@@ -995,17 +995,20 @@ __device__ __forceinline__ void q4k_matmul_rm(const uint8_t *__restrict__ q,
 // groups idle for a round and make the others' sums longer (14336 x 1536 x 128
 // error 1.40e-7 against 1.33e-7 in 64 bits, now 1.32e-7).
 //
-// What bounds it: the vector unit's issue slots.  A 32x32x16 MFMA is 35 cycles
-// of the matrix core and its 5 VALU instructions of dequantisation (at 128
-// columns; 20 at 32) take 4 to 5 cycles each beside it, for two waves per
-// SIMD; at 512 columns the card's power adds to that (the clock falls from 2.4
-// to 1.8 GHz, and a copy of the kernel without its waits takes as long).
+// What bounds it, by counters at 14336 x 4096 and 64, 128, 256, 512 columns: the
+// matrix cores are busy 12, 19, 31 and 39% of the cycles, and the other vector
+// instructions (14, 7, 6 and 6 for every MFMA, 11, 5, 5 and 5 of them
+// dequantisation) would fill 21, 16, 23 and 28% at four cycles each, so even one
+// after the other the two leave a third to two thirds; the waves wait 28 to 34%
+// of their time for a counter or a barrier and as long for an instruction to
+// issue.  No LDS bank conflicts.
 // Measured against the bodies it replaced (four waves, 64-wide chunks dealt
 // out to K groups or whole rows, headers decoded per chunk), same tiles, us:
 // 14336 x 4096 x 512 75.4 -> 68.4, x 256 42 -> 36.5, x 64 20.6 -> 18.2, x 128
 // 27.4 -> 26.4; 28672 x 14336 x 256 265 -> 217; 4096 x 14336 x 128 44.5 -> 36;
 // 5000 x 11008 x 77 36.4 -> 29.1 with the f32 cast.  Errors against 64 bits
-// are the same, or lower where K is split in more groups than before.
+// are the same within the order of the sums (5000 x 11008 x 77 3.35e-7 against
+// 3.33e-7, 14336 x 4096 x 512 4.1e-7 both).
 // ---------------------------------------------------------------------------
 template <int KQ, int CT>
 __device__ __forceinline__ void q4k_matmul_wk(const uint8_t *__restrict__ q,
@@ -1727,8 +1730,8 @@ AXH_Q4K_MATMUL_WK(1, 4, rm_w8_r1_p4)
 
 // Two kernels have a second body, 32 rows x 32 columns with K in 8, which the
 // host selects by shape (a.pad = 1, see matmul_launch_of): past one 16-row
-// block per workgroup (streaming rows) and past 16 columns (one-column-tile
-// K-split tiles, whose four waves let the other four end at once).
+// block per workgroup (streaming rows) and past 16 columns of enough superblocks
+// (one-column-tile K-split tiles, whose four waves let the other four end at once).
 extern "C" __global__ void __launch_bounds__(512)
     axh_q4k_matmul_sr_w8_s2_n2(const uint8_t *__restrict__ q, const uint16_t *__restrict__ x,
                                float *__restrict__ y, AXH_MATMUL_ARGS) {
