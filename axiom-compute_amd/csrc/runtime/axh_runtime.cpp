@@ -585,10 +585,12 @@ static axh_status dispatch_staged(axh_context *ctx, axh_kernel *k, const uint32_
   axh_status s = builtin_kernel(ctx, "axh_copy_segments", 1, 4, 256, &copy);
   if (s != AXH_OK) return s;
   hipError_t e = hipSuccess;
-  // Waits for all of it; a timeout leaves copies queued on the staging buffer.
+  // Waits for all of it; a wait that fails, by a timeout or otherwise, leaves
+  // copies queued on the staging buffer, if any came that far.
+  bool queued = false;
   auto finish = [&]() {
     const axh_status st = wait_stream(core, core.stream);
-    *busy = st == AXH_ERR_FENCE_TIMEOUT;
+    *busy = queued && st != AXH_OK;
     return st;
   };
   // An error in between leaves what was queued before it: once that is done the
@@ -604,7 +606,10 @@ static axh_status dispatch_staged(axh_context *ctx, axh_kernel *k, const uint32_
     const size_t wgs = (largest + 4095) / 4096; // 16 bytes per thread of a workgroup
     const uint32_t grid[3] = {(uint32_t)(wgs < 1 ? 1 : wgs > kCopyWgs ? kCopyWgs : wgs), segs, 1};
     void *bufs[1] = {table};
-    return launch_raw(copy, grid, bufs, 1, &segs, sizeof(segs), 0, core.stream);
+    const axh_status st =
+        launch_raw(copy, grid, bufs, 1, &segs, sizeof(segs), 0, core.stream);
+    queued |= st == AXH_OK;
+    return st;
   };
   CopySegment *tin = static_cast<CopySegment *>(staging), *tout = tin + n;
   uint8_t *at = static_cast<uint8_t *>(staging) + staged_size(2 * n * sizeof(CopySegment));
@@ -622,6 +627,7 @@ static axh_status dispatch_staged(axh_context *ctx, axh_kernel *k, const uint32_
         return drop(fail(AXH_ERR_STAGING_COPY, "binding #" + std::to_string(i) +
                                                    " (HostToDevice): " +
                                                    hip_msg("hipMemcpyAsync", e)));
+      queued = true;
     }
     at += staged_size(input_sizes[i]);
   }
@@ -642,6 +648,7 @@ static axh_status dispatch_staged(axh_context *ctx, axh_kernel *k, const uint32_
       if (e != hipSuccess)
         return drop(fail(AXH_ERR_READBACK, "readback of binding #" + std::to_string(i) +
                                                " failed: " + hip_msg("hipMemcpyAsync", e)));
+      queued = true;
     }
     at += staged_size(output_sizes[i]);
   }

@@ -131,8 +131,8 @@ uint64_t axh_kernel_pool_bytes(const axh_kernel *k, uint32_t binding);
  * 32 MiB in all go through one pinned buffer each, taken from the context for
  * the call: it keeps up to 8 of them and 64 MiB between calls, for all its
  * handles, until it is destroyed (besides the one of up to 32 MiB that larger
- * requests, uploads and downloads share).  A request that times out keeps its
- * buffer until then. */
+ * requests, uploads and downloads share).  A request whose wait
+ * fails (a timeout) keeps its buffer until then. */
 axh_status axh_dispatch_handle(axh_context *ctx, axh_kernel *k, const uint32_t workgroups[3],
                                const void *const *inputs, const size_t *input_sizes,
                                size_t n_inputs, const size_t *output_sizes, size_t n_outputs,

@@ -76,6 +76,37 @@ def test_dispatch_after_a_timed_out_one(axc):
     ctx.close()
 
 
+def test_buffer_of_a_wait_that_failed(axc):
+    """A request made while the stream records a graph cannot wait: its copies are
+    recorded or queued, not done, so its buffer is not used again.  The requests
+    after it fail before anything is queued (the recording is invalid) and share
+    the next buffer."""
+    print("dispatch during a capture", flush=True)
+    ctx = axc.HipContext.new_with_options(axc.HipContextOptions(fence_timeout_ms=5000))
+    h = np.random.default_rng(5).integers(0, 0x7C00, 4 << 20).astype(np.uint16)  # 8 MiB
+    k = ctx.prepare_kernel(axc.builtin_code_object(), _plan(axc, 2, 4, 256), 4, "axh_f16_widen")
+
+    def request():
+        return ctx.dispatch_handle(k, (1, 1, 1), [h.tobytes(), b""], [0, 1024],
+                                   struct.pack("<I", 256))
+
+    want = h[:256].view(np.float16).astype(np.float32).tobytes()
+    assert request()[1] == want  # leaves its 16 MiB buffer idle
+    with pytest.raises(axc.DispatchError) as e:
+        ctx.capture(request)
+    assert e.value.variant == "QueueSubmitFailed"
+    before = _address_space()
+    for _ in range(3):
+        with pytest.raises(axc.DispatchError) as e:
+            request()
+        assert e.value.variant == "StagingCopyFailed"
+    grown = _address_space() - before
+    print(f"  address space grew by {grown >> 20} MiB", flush=True)
+    assert 16 << 20 <= grown < 32 << 20
+    k.release()
+    ctx.close()
+
+
 def test_handles_share_their_pinned_memory(axc):
     """Eight live handles, each with a request of 8 MiB: one staging buffer of 16
     MiB, not one for each (which a handle held for its life)."""
