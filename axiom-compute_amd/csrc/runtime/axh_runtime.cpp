@@ -135,13 +135,13 @@ static axh_status ensure_staging(Core &core, size_t bytes) {
 
 static constexpr size_t kStagingChunk = size_t(32) << 20;
 
-// A wait that timed out leaves its copy queued on the stream, still reading
-// or writing the staging buffer.  The buffer is retired (freed when the core
-// goes away) so the next staged copy fills a fresh one instead of handing
-// the queued transfer the wrong bytes.
+// A wait that timed out, or that failed before it saw the stream drain, leaves
+// its copy queued, still reading or writing the staging buffer.  The buffer is
+// retired (freed when the core goes away) so the next staged copy fills a fresh
+// one instead of handing the queued transfer the wrong bytes.
 static axh_status staging_wait(Core &core) {
   const axh_status s = wait_stream(core, core.stream);
-  if (s == AXH_ERR_FENCE_TIMEOUT && core.staging) {
+  if (s != AXH_OK && core.staging) {
     core.retired_staging.push_back(core.staging);
     core.staging = nullptr;
     core.staging_bytes = 0;

@@ -107,6 +107,28 @@ def test_buffer_of_a_wait_that_failed(axc):
     ctx.close()
 
 
+def test_staging_of_a_copy_whose_wait_failed(axc):
+    """The same for the staging memory that uploads and downloads share."""
+    print("upload during a capture", flush=True)
+    ctx = axc.HipContext.new_with_options(axc.HipContextOptions(fence_timeout_ms=5000))
+    data = np.random.default_rng(6).integers(0, 256, 8 << 20).astype(np.uint8)
+    buf = ctx.alloc(data.nbytes)
+    ctx.upload(buf, data)
+    with pytest.raises(axc.DispatchError) as e:
+        ctx.capture(lambda: ctx.upload(buf, data))
+    assert e.value.variant == "QueueSubmitFailed"
+    before = _address_space()
+    for _ in range(3):
+        with pytest.raises(axc.DispatchError) as e:
+            ctx.upload(buf, data)
+        assert e.value.variant == "StagingCopyFailed"
+    grown = _address_space() - before
+    print(f"  address space grew by {grown >> 20} MiB", flush=True)
+    assert 8 << 20 <= grown < 16 << 20
+    buf.close()
+    ctx.close()
+
+
 def test_handles_share_their_pinned_memory(axc):
     """Eight live handles, each with a request of 8 MiB: one staging buffer of 16
     MiB, not one for each (which a handle held for its life)."""
