@@ -58,3 +58,31 @@ def test_rows_equal_those_of_smaller_calls(ctx, axc, fmt, rows, units):
 def test_defaults(axc, fmt, rows, units, one):
     name = getattr(axc, fmt + "_matvec_kernel_name")(rows, units)
     assert name.startswith(f"axh_{fmt}_matvec_{'one_' if one else 'flat_'}")
+
+
+def test_first_use_while_recording(axc):
+    """The wide kernels are a code object of their own: a context that has not
+    launched one yet can load it while its stream records."""
+    print("wide one-pass kernel first used in a capture", flush=True)
+    rows, units = 4999, 3
+    c = axc.HipContext.new()
+    q = O.gen_q4k_weights(11, rows * units)
+    x = O.gen_normal_f32(12, units * 256)
+    dq, dx, dy, de = c.alloc(q.nbytes), c.alloc(x.nbytes), c.alloc(rows * 4), c.alloc(rows * 4)
+    c.upload(dq, q)
+    c.upload(dx, x)
+    g = c.capture(lambda: c.q4k_matvec(dq, dx, dy, rows, units))
+    for _ in range(3):
+        c.upload(dy, np.full(rows, np.nan, dtype=np.float32))
+        c.upload(de, np.full(rows, np.nan, dtype=np.float32))
+        c.q4k_matvec(dq, dx, de, rows, units)
+        c.synchronize()
+        g.launch()
+        c.synchronize()
+        got = c.download(dy, rows * 4)
+        assert got == c.download(de, rows * 4)
+        assert not np.isnan(np.frombuffer(got, dtype=np.float32)).any()
+    g.close()
+    for b in (dq, dx, dy, de):
+        b.close()
+    c.close()
