@@ -1660,6 +1660,7 @@ AXH_Q4K_MATMUL_KS(8, 1, 2, 1, _r1)
     q4k_matmul_kx<RT, NT, KS, PF>(q, x, y, a, axh_red_dyn);                                      \
   }
 
+AXH_Q4K_MATMUL_KX(4, 1, 4, 3, )
 AXH_Q4K_MATMUL_KX(2, 8, 4, 2, )
 AXH_Q4K_MATMUL_KX(4, 4, 4, 3, )
 AXH_Q4K_MATMUL_KX(8, 4, 4, 2, )
@@ -1691,6 +1692,7 @@ AXH_Q4K_MATMUL_RM(4, 1, _short)
   }
 
 AXH_Q4K_MATMUL_SR(8, 2, 1, false, )
+AXH_Q4K_MATMUL_SR(8, 2, 2, false, _n2)
 AXH_Q4K_MATMUL_SR(8, 2, 1, true, _h)
 
 #define AXH_Q4K_MATMUL_LK(XC, XD, WD, RT, SUFFIX)                                               \
@@ -1728,28 +1730,20 @@ AXH_Q4K_MATMUL_WK(4, 4, kx_r4_n8_k4_p2)
 AXH_Q4K_MATMUL_WK(2, 4, rm_w4_r1_p4)
 AXH_Q4K_MATMUL_WK(1, 4, rm_w8_r1_p4)
 
-// Two kernels have a second body, 32 rows x 32 columns with K in 8, which the
-// host selects by shape (a.pad = 1, see matmul_launch_of): past one 16-row
-// block per workgroup (streaming rows) and past 16 columns of enough superblocks
-// (one-column-tile K-split tiles, whose four waves let the other four end at once).
-extern "C" __global__ void __launch_bounds__(512)
-    axh_q4k_matmul_sr_w8_s2_n2(const uint8_t *__restrict__ q, const uint16_t *__restrict__ x,
-                               float *__restrict__ y, AXH_MATMUL_ARGS) {
-  AXH_MATMUL_UNPACK;
-  extern __shared__ f32x4_t axh_sr_dyn[];
-  if (__builtin_expect(a.pad == 0u, 1))
-    q4k_matmul_sr<8, 2, 2, false>(q, x, y, a, axh_sr_dyn);
-  else
-    q4k_matmul_wk<8, 1>(q, x, y, a, axh_sr_dyn);
-}
-
+// 32 rows x 32 columns with K in 8, one kernel for two variants that the host
+// leaves for it by shape (see matmul_launch_of): streaming rows of 32 columns past
+// one 16-row block per CU, and 64 x 16 K-split tiles past 16 columns.  As a second
+// body of those kernels it cost their first ones registers and schedule: at 104
+// VGPRs for 76, and 512 threads of which half ended at once, 9000 x 4608 x 6 took
+// 14.1 us against 13.7, 12086 x 5376 x 1 16.1 against 15.9.  It gained by the
+// change where it stands for streaming rows (4096 x 1024 x 64 5.66 -> 5.50 us, 1024
+// x 4096 x 250 7.99 -> 7.81) and lost up to 1.3% elsewhere (8000 x 8192 x 24 13.97 ->
+// 14.15), less than without the register limit (at most 128: 8192 x 14336 x 32 24.9
+// against 25.1).
 extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
-    axh_q4k_matmul_kx_r4_n1_k4_p3(const uint8_t *__restrict__ q, const uint16_t *__restrict__ x,
-                                  float *__restrict__ y, AXH_MATMUL_ARGS) {
+    axh_q4k_matmul_t32(const uint8_t *__restrict__ q, const uint16_t *__restrict__ x,
+                       float *__restrict__ y, AXH_MATMUL_ARGS) {
   AXH_MATMUL_UNPACK;
-  extern __shared__ f32x4_t axh_kx1_dyn[];
-  if (a.pad != 0u)
-    q4k_matmul_wk<8, 1>(q, x, y, a, axh_kx1_dyn);
-  else if (threadIdx.x < 256u)
-    q4k_matmul_kx<4, 1, 4, 3>(q, x, y, a, axh_kx1_dyn);
+  extern __shared__ f32x4_t axh_t32_dyn[];
+  q4k_matmul_wk<8, 1>(q, x, y, a, axh_t32_dyn);
 }

@@ -48,9 +48,9 @@ struct MatmulArgs {
 //                       register A, operands through per-wave LDS rings, PF superblocks in
 //                       flight.  r4 with n2, n4 p2 and n8 p2 (from 8 superblocks) and kind
 //                       8's r1 (from 6 at W = 4) run the wide-K-step body of 8 waves
-//                       (matmul_wide); n1 past 16 columns and kind 7's _n2 between one and
-//                       two blocks per CU its 32 x 32 form, where that is ahead
-//                       (matmul_launch_of).
+//                       (matmul_wide); for n1 past 16 columns and kind 7's _n2 between one
+//                       and two blocks per CU its 32 x 32 form is launched, where that is
+//                       ahead (axh_q4k_matmul_t32, see matmul_launch_of).
 //   kind 7 (streaming rows) axh_q4k_matmul_sr_w{W}_s2[_n2|_h]: persistent, one workgroup per
 //                       CU over 16-row blocks, K <= 4096 (pf 2: 8-column groups).
 //   kind 8 (32x32 tiles) axh_q4k_matmul_rm_w{W}_r{RT}_p4: W waves of RT 32-row MFMA tiles
@@ -1733,9 +1733,11 @@ static bool matmul_short(const MatmulVariant &v, uint32_t n_rows, uint32_t batch
 }
 
 // What a matmul variant launches for a shape: outputs per workgroup, threads,
-// LDS, and whether its kernel runs its second body.
+// LDS, and whether the 32 x 32 tiles of axh_q4k_matmul_t32 take the place of the
+// variant's own kernel.
 struct MatmulLaunch {
-  uint32_t rows, cols, threads, lds, second;
+  uint32_t rows, cols, threads, lds;
+  bool t32;
 };
 
 static MatmulLaunch matmul_launch_of(const MatmulVariant &v, uint32_t n_rows, uint32_t batch,
@@ -1756,11 +1758,11 @@ static MatmulLaunch matmul_launch_of(const MatmulVariant &v, uint32_t n_rows, ui
     // the grid (4096 x 4096 x 64 9.1 us against 12.4, 4096 x 1024 x 64 6.1
     // against 10.4, 1024 x 4096 x 250 8.8 against 12.0, A/B in one run); not
     // before (4096 x 4096 x 32 8.6 against 7.3).  With one column group (4097
-    // to 8192 rows, up to 32 columns) the first body reads X once for all of a
+    // to 8192 rows, up to 32 columns) the streaming kernel reads X once for all of a
     // CU's blocks, and the tiles are ahead only where their 8 K groups come out
     // even: 5000 rows x 24 columns, K = 1024, 1536, 1792, 2048, 2304, 3072, 3840,
-    // 4096: 0.89, 1.00, 1.09, 0.90, 1.04, 1.17, 1.33, 1.14 times the first
-    // body's time (3072: 8.31 us against 6.99; weights rotated through 0.4 to
+    // 4096: 0.89, 1.00, 1.09, 0.90, 1.04, 1.17, 1.33, 1.14 times its time
+    // (3072: 8.31 us against 6.99; weights rotated through 0.4 to
     // 1 GB 0.87, 0.97, 1.06, 0.91, 1.03, 1.16, 1.33, 1.11).
     if (groups(16, 32) > kMatmulCus && groups(32, 32) <= kMatmulCus &&
         (batch > 32 || nsb <= 6 || nsb == 8))
@@ -1777,11 +1779,10 @@ static MatmulLaunch matmul_launch_of(const MatmulVariant &v, uint32_t n_rows, ui
     if (batch > 16 && nsb >= 8 &&
         (groups(32, 32) <= kMatmulCus || nsb >= (half_empty ? 32u : 16u)))
       k_groups = 8;
-    l.threads = 512; // the kernel's; four of the waves end at once
   }
   if (k_groups == 8) {
     l.rows = l.cols = 32;
-    l.second = 1;
+    l.t32 = true;
   }
   if (k_groups) {
     l.threads = 512;
@@ -1882,7 +1883,7 @@ static MatmulVariant q4k_matmul_default(uint32_t n_rows, uint32_t batch, uint32_
     return groups(128, 128) > kMatmulCus ? MatmulVariant{8, 8, 8, 4, 1}
                                          : MatmulVariant{8, 4, 8, 4, 1};
   // Kind 5 beyond: the narrowest of its tiles whose grid is one round, since a
-  // second round doubles the time whatever it holds.  32 x 32 (the second body
+  // second round doubles the time whatever it holds.  32 x 32 (t32 in place
   // of the one-column-tile kernel): 4096 x 14336 x 64 22 us against 39 as 64 x
   // 16 and 47 in 64 x 32 tiles, 8192 x 14336 x 32 25.7 against 42.  64 x 32
   // while they fit: 5000 x 11008 x 77 30 us against 35 in 64 x 64 tiles.  64 x
@@ -2046,13 +2047,14 @@ axh_status axh_q4k_matmul_f16(axh_context *ctx, const void *q, const uint16_t *x
     return fail(AXH_ERR_WORKGROUP_COUNT_EXCEEDS_LIMIT, "matmul grid exceeds the device limit");
   hipSetDevice(ctx->core->device);
   axh_kernel *k = nullptr;
-  s = builtin_kernel(ctx, name, 3, sizeof(MatmulArgs), l.threads, &k);
+  s = builtin_kernel(ctx, l.t32 ? "axh_q4k_matmul_t32" : name, 3, sizeof(MatmulArgs), l.threads,
+                     &k);
   if (s != AXH_OK) return s;
   // kind 7 is persistent: one workgroup per CU per column group, even where two would fit
-  if (v.kind == 7 && !l.second && ctx->core->cu_count < gx) gx = ctx->core->cu_count;
+  if (v.kind == 7 && !l.t32 && ctx->core->cu_count < gx) gx = ctx->core->cu_count;
   const uint32_t grid[3] = {(uint32_t)gx, (uint32_t)gy, 1};
   void *bufs[3] = {const_cast<void *>(q), const_cast<uint16_t *>(x), y};
-  MatmulArgs a{n_rows, sb_per_row, batch, l.second};
+  MatmulArgs a{n_rows, sb_per_row, batch, 0};
   s = launch_raw(k, grid, bufs, 3, &a, sizeof(a), l.lds, pick_stream(ctx, stream));
   return s == AXH_OK ? ok() : s;
 }

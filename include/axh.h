@@ -506,6 +506,8 @@ axh_status axh_q4k_matmul_f16(axh_context *ctx, const void *q, const uint16_t *x
 axh_status axh_q4k_matmul_f32(axh_context *ctx, const void *q, const float *x, uint16_t *x16,
                               float *y, uint32_t n_rows, uint32_t sb_per_row, uint32_t batch,
                               const axh_q4_matmul_variant *variant, void *stream);
+/* The name of the variant's kernel; where 32 x 32 tiles take its place (kind 7
+ * with 32 columns, kind 5 with 16) a trace shows axh_q4k_matmul_t32. */
 axh_status axh_q4k_matmul_kernel_name(uint32_t n_rows, uint32_t sb_per_row, uint32_t batch,
                                       const axh_q4_matmul_variant *variant, char *buf,
                                       size_t cap);

@@ -2,6 +2,7 @@
 own metadata (no GPU needed)."""
 from __future__ import annotations
 
+import ctypes
 import re
 import struct
 
@@ -35,3 +36,17 @@ def test_one_pass_matvecs_are_compiled_for_eight_waves(axc):
     assert {k[".max_flat_workgroup_size"] for k in one.values()} == {512}
     assert not any(k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]
                    for k in one.values())
+
+
+def test_matmul_kernels_hold_one_body(axc):
+    """The 32 x 32 tiles that take the place of other variants' kernels are a kernel
+    of their own: as a second body they cost the first ones their launch size of
+    four waves and a third more registers."""
+    lib = axc.load_library()
+    begin, end = (ctypes.addressof(ctypes.c_char.in_dll(lib, f"axh_q4_matmul_co_{n}"))
+                  for n in ("begin", "end"))
+    kernels = _kernels(ctypes.string_at(begin, end - begin))
+    assert kernels["axh_q4k_matmul_t32"][".max_flat_workgroup_size"] == 512
+    assert kernels["axh_q4k_matmul_kx_r4_n1_k4_p3"][".max_flat_workgroup_size"] == 256
+    # 6 waves per SIMD (512 VGPRs), against 4 with both bodies
+    assert kernels["axh_q4k_matmul_kx_r4_n1_k4_p3"][".vgpr_count"] <= 80
