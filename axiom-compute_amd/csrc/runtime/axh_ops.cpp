@@ -1878,7 +1878,10 @@ static MatmulVariant q4k_matmul_default(uint32_t n_rows, uint32_t batch, uint32_
   // 128 ones are one round: 8192 x 4096 x 256 25.8 us in 256 of them against
   // 30.1, but 8193 rows 44.0 against 33.9, 9216 x 4096 x 256 41.5 against 30.5,
   // 18432 x 4096 x 128 43.7 against 31.3, 4608 x 4096 x 512 41.5 against 31.0,
-  // 10112 x 14336 x 256 133 against 97, 9216 x 768 x 256 18.5 against 11.1.
+  // 10112 x 14336 x 256 133 against 97, 9216 x 768 x 256 18.5 against 11.1.  There
+  // K is in two sums instead of four: error against 64 bits 2.3e-7 for 1.7e-7 at
+  // 9964 x 2560 x 139 (10777 x 4864 x 137, as before 128-row tiles: 3.1e-7, and
+  // 4.4e-7 when those had all of K in one sum).
   if (batch >= 128 && (groups(128, 128) >= kMatmulFill || groups(64, 128) > kMatmulCus))
     return groups(128, 128) > kMatmulCus ? MatmulVariant{8, 8, 8, 4, 1}
                                          : MatmulVariant{8, 4, 8, 4, 1};
