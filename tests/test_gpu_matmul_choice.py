@@ -1,4 +1,5 @@
-"""Which body the batched matmul's kernels with two bodies run (marked `gpu`).
+"""Where 32 x 32 tiles take the place of a batched matmul variant's own kernel, and
+where the narrow-step bodies run (marked `gpu`).
 
 A body forms every output from its row's weights and its column's activations
 in an order of its own, whatever the size of the grid, so an output equals,
@@ -39,7 +40,7 @@ class _Data:
             b.close()
 
 
-# 16 columns: 64 x 16 tiles, the first body of the one-column-tile kernel
+# 16 columns: 64 x 16 tiles, the one-column-tile kernel's own
 @pytest.mark.parametrize("rows,sb,batch,tiles", [
     (300, 1, 48, False), (300, 7, 64, False), (300, 8, 33, True),      # one round of 32 x 32
     (8224, 7, 17, False), (8224, 12, 64, False), (8224, 15, 32, False),  # more than one
@@ -82,7 +83,7 @@ def test_two_column_tiles_in_rounds(ctx, axc, rows, sb, batch, kernel):
     assert np.array_equal(whole[:16], narrow) == kernel.endswith("_short")
 
 
-# 4096 rows of up to 32 columns: one 16-row block per CU, the first body
+# 4096 rows of up to 32 columns: one 16-row block per CU, the variant's own kernel
 @pytest.mark.parametrize("rows,sb,batch,tiles", [
     (4097, 6, 17, True), (5000, 7, 24, False), (5000, 8, 24, True), (5000, 9, 24, False),
     (5000, 12, 24, False), (8192, 15, 17, False), (8192, 16, 32, False)])

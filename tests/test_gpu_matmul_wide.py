@@ -91,7 +91,7 @@ def test_short_and_wide_steps(ctx, axc, rows, sb, variant, kernel):
 
 
 def test_streaming_rows_second_body_line(ctx, axc):
-    """One 16-row block per CU stays with the first body; a second block per CU
+    """One 16-row block per CU stays with the variant's own kernel; a second block per CU
     goes to 32-row tiles while those are one round, in every K remainder (4097
     rows of 32 columns, one column group: only where K splits evenly)."""
     for rows, sb, batch in [(4096, 16, 32), (4097, 16, 32), (2064, 7, 64), (1024, 1, 250)]:
